@@ -466,7 +466,7 @@ def lm_head_argmax(x, w_packed, vocab, rows=None, want_logits=False, workspace=N
 
 def sample_rows(logits, temp, top_k=0, top_p=1.0, draft=None, u=None, want_p_draft=False, want_draw=False,
                 want_probs=False):
-    """Temperature / top-k / top-p over bf16 logits rows [R, V] (one workgroup per row).  draft int32 [R]
+    """Temperature / top-k / top-p over bf16 logits rows [R, V].  draft int32 [R]
     (device, -1 = none) and u float64 [R] (device uniforms in [0, 1)) are optional; returns a dict with
     the requested outputs: p_draft fp32 [R], draw int32 [R] (needs u unless temp <= 0), probs fp32 [R, V]."""
     R, V = logits.shape
@@ -485,9 +485,10 @@ def sample_rows(logits, temp, top_k=0, top_p=1.0, draft=None, u=None, want_p_dra
         out["draw"] = torch.empty(R, dtype=torch.int32, device=dev)
     if want_probs:
         out["probs"] = torch.empty(R, V, dtype=torch.float32, device=dev)
-    check(lib().flyai_sample_rows(_ptr(logits), R, V, float(temp), int(top_k), float(top_p), _ptr(draft), _ptr(u),
-                                  _ptr(out.get("p_draft")), _ptr(out.get("draw")), _ptr(out.get("probs")),
-                                  _stream()))
+    ws = torch.empty(int(lib().flyai_sample_workspace_bytes(R, V)), dtype=torch.uint8, device=dev)
+    check(lib().flyai_sample_rows_ws(_ptr(logits), R, V, float(temp), int(top_k), float(top_p), _ptr(draft), _ptr(u),
+                                     _ptr(out.get("p_draft")), _ptr(out.get("draw")), _ptr(out.get("probs")),
+                                     _ptr(ws), _stream()))
     return out
 
 

@@ -352,6 +352,12 @@ int flyai_hbm_read_probe(const void* src, size_t bytes, int32_t nontemporal, int
 int flyai_sample_rows(const uint16_t* logits, int32_t R, int32_t V, float temp, int32_t top_k, float top_p,
                       const int32_t* draft, const double* u, float* p_draft, int32_t* draw, float* probs,
                       flyai_stream_t stream);
+/* flyai_sample_rows with a device workspace (8-byte aligned, flyai_sample_workspace_bytes(R, V) bytes, not
+ * initialised): the same results bit for bit, each row split over many workgroups. */
+size_t flyai_sample_workspace_bytes(int32_t R, int32_t V);
+int flyai_sample_rows_ws(const uint16_t* logits, int32_t R, int32_t V, float temp, int32_t top_k, float top_p,
+                         const int32_t* draft, const double* u, float* p_draft, int32_t* draw, float* probs,
+                         void* workspace, flyai_stream_t stream);
 /* A draw from a probability vector p[V] (fp32, device; Sampler.sample): weights floor(p * 2^40), then the
  * same inverse-CDF rule with uniform u in [0, 1); out (device int32) gets the id (0 when all are 0). */
 int flyai_sample_probs(const float* probs, int32_t V, double u, int32_t* out, flyai_stream_t stream);

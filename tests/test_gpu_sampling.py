@@ -189,3 +189,42 @@ def test_sample_rows_non_finite_logits_and_out_of_range_uniforms(bad):
             assert np.array_equal(probs[r], S.probs(w)), r
         else:
             assert not probs[r].any(), r
+
+
+CHUNKED = [  # (rows, V, temp, top_k, top_p): ids per chunk 4096 up to 262,144 ids, then a multiple of 2048
+    (3, 4096, 0.8, 0, 0.9), (3, 4097, 1.0, 40, 1.0), (2, 8191, 1.1, 40, 0.9), (2, 16392, 0.7, 3, 0.5),
+    (5, V_GPTOSS, 1.2, 0, 0.95), (2, V_GPTOSS, 0.9, 200, 0.9), (2, 262153, 0.9, 0, 0.97), (300, 4104, 0.9, 5, 0.9),
+]
+
+
+@pytest.mark.parametrize("R,V,temp,top_k,top_p", CHUNKED)
+def test_split_rows_equal_one_workgroup_rows(R, V, temp, top_k, top_p):
+    """The rows split over workgroups (a workspace) against one workgroup a row (no workspace), bit for bit:
+    ragged last chunks, odd row lengths (no vector loads), ties across chunks at the top-k and top-p
+    boundaries, drafted tokens inside the ties, -inf masks, and rows for the general path (NaN, +inf,
+    quotients near the denormals, an overflowing temperature)."""
+    import ctypes as C
+    from flyai_amd import _lib, ops
+    x = _logits(R, V, seed=V + R, ties=True)
+    if R >= 2:
+        x[1, :V // 2] = float("-inf")                 # masked vocabulary
+        x[1, V // 3] = 1e-36                           # a quotient near the denormals
+    if R >= 3:
+        x[2] = 1.25                                    # one tie over the whole row
+    if R >= 5:
+        x[3, 11], x[4, 7], x[4, 8] = float("nan"), 3e38, float("-inf")
+    g = torch.Generator().manual_seed(V)
+    d = torch.randint(-1, V, (R,), generator=g, dtype=torch.int32)
+    d[0] = int(x[0].float().argmax())
+    u = torch.rand(R, generator=g, dtype=torch.float64)
+    xd, dd, ud = x.to(DEV), d.to(DEV), u.to(DEV)
+    for t in (temp, 1e-30, 0.0):
+        got = ops.sample_rows(xd, t, top_k, top_p, draft=dd, u=ud, want_p_draft=True, want_draw=True, want_probs=True)
+        want = {n: torch.empty_like(v) for n, v in got.items()}
+        p = lambda v: C.c_void_p(v.data_ptr())  # noqa: E731
+        _lib.check(_lib.lib().flyai_sample_rows(p(xd), R, V, t, top_k, top_p, p(dd), p(ud), p(want["p_draft"]),
+                                                p(want["draw"]), p(want["probs"]),
+                                                C.c_void_p(torch.cuda.current_stream().cuda_stream)))
+        torch.cuda.synchronize()
+        for n in got:
+            assert torch.equal(got[n], want[n]), (t, n, (got[n] != want[n]).nonzero()[:4].tolist())
