@@ -83,6 +83,17 @@ struct TreeView {
   const uint64_t* mask = nullptr;
 };
 
+__device__ __forceinline__ TreeView tree_view(const flyai_attn_tree* tree, int window) {
+  const char* tb = reinterpret_cast<const char*>(tree);
+  TreeView tv;
+  tv.start = tree->start;
+  tv.n = tree->n_nodes;
+  tv.words = tree->words;
+  tv.depth = reinterpret_cast<const int32_t*>(tb + tree->depth_off);
+  tv.mask = reinterpret_cast<const uint64_t*>(tb + tree->mask_off[window > 0 ? 1 : 0]);
+  return tv;
+}
+
 // Per-wave state of QT query-row tiles of 16 (QT = 1: up to 2 tokens; QT = 2: up to 4 tokens): the
 // Q^T operand, each row's position (and, in a tree, its depth and node), and the running
 // softmax (max, sum, O^T accumulators).  Query row rq = 16*qt + n is token rq/8, head kv_head*8 + rq%8.
@@ -160,13 +171,64 @@ __device__ __forceinline__ float max_lane_groups(float v) {
 constexpr float kMaxSlack = 8.f;
 constexpr float kMaxSentinel = -1e29f;  // a running max at or below this is the initial -1e30 (no key yet)
 
+// The scores s of one 64-key block and row tile qt: keys outside the row's range become -inf; returns each
+// row's largest (all four lane groups hold it).
+template <int QT, bool TREE>
+__device__ __forceinline__ float rows_mask_max(const QRows<QT>& R, f32x4_t (&s)[4], int qt, int kb, bool interior,
+                                               int key_lo, int key_hi, int window, const TreeView& tv) {
+  const int g = (threadIdx.x & 63) >> 4;
+  const int tstart = TREE ? tv.start : 0;
+  // lane holds S^T[key kb + tile_key(kt, 4g + v)][qrow n]
+  float bmax = -INFINITY;
+  if (interior && R.qval[qt]) {
+#pragma unroll
+    for (int kt = 0; kt < 4; ++kt)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) bmax = fmaxf(bmax, s[kt][v]);
+  } else {
+    const int p = R.qpos[qt];
+    const int lo = max(key_lo, window > 0 ? p - window + 1 : 0);
+    const int hi = min(p, key_hi - 1);
+    // tree: bits [kb - start, kb - start + 64) of the row's mask (key kb + t is bit t)
+    uint64_t tbits = 0;
+    if (TREE) {
+      const int j0 = kb - tstart;
+      if (R.qval[qt] && j0 > -64 && j0 < tv.n) {
+        const int wq = j0 >> 6, sh = j0 & 63;  // floor division (j0 may be negative)
+        const uint64_t* mrow = tv.mask + (size_t)R.qnode[qt] * tv.words;
+        const uint64_t w0 = wq >= 0 ? mrow[wq] : 0ull;
+        const uint64_t w1 = wq + 1 < tv.words ? mrow[wq + 1] : 0ull;
+        tbits = sh == 0 ? w0 : (w0 >> sh) | (w1 << (64 - sh));
+      }
+    }
+#pragma unroll
+    for (int kt = 0; kt < 4; ++kt)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        const int key = kb + tile_key(kt, 4 * g + v);
+        bool ok;
+        if (TREE) {
+          if (key < tstart)
+            ok = key >= lo && key < key_hi;  // committed prefix (window on positions)
+          else  // tree slot: the mask (its window already applied for sliding layers)
+            ok = key >= key_lo && key < key_hi && ((tbits >> tile_key(kt, 4 * g + v)) & 1ull);
+          ok = ok && R.qval[qt];
+        } else {
+          ok = R.qval[qt] && key >= lo && key <= hi;
+        }
+        s[kt][v] = ok ? s[kt][v] : -INFINITY;
+        bmax = fmaxf(bmax, s[kt][v]);
+      }
+  }
+  return max_lane_groups(bmax);
+}
+
 template <int QT, bool TREE>
 __device__ __forceinline__ void rows_block(QRows<QT>& R, const uint4 (&kc)[4][2], uint4 (&vv)[4][2], int kb,
                                            bool interior, int key_lo, int key_hi, int window,
                                            const TreeView& tv) {
   const int g = (threadIdx.x & 63) >> 4;
   const float scale = 0.125f * kLog2e;
-  const int tstart = TREE ? tv.start : 0;
   const bf16x8_t ones = as_bf16x8(make_uint4(0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u));
   if (kb + 64 > key_hi) {
 #pragma unroll
@@ -182,49 +244,7 @@ __device__ __forceinline__ void rows_block(QRows<QT>& R, const uint4 (&kc)[4][2]
       s[kt] = mfma16x16x32(as_bf16x8(kc[kt][0]), R.qf[qt][0], f32x4_t{0.f, 0.f, 0.f, 0.f});
       s[kt] = mfma16x16x32(as_bf16x8(kc[kt][1]), R.qf[qt][1], s[kt]);
     }
-    // lane holds S^T[key kb + tile_key(kt, 4g + v)][qrow n]
-    float bmax = -INFINITY;
-    if (interior && R.qval[qt]) {
-#pragma unroll
-      for (int kt = 0; kt < 4; ++kt)
-#pragma unroll
-        for (int v = 0; v < 4; ++v) bmax = fmaxf(bmax, s[kt][v]);
-    } else {
-      const int p = R.qpos[qt];
-      const int lo = max(key_lo, window > 0 ? p - window + 1 : 0);
-      const int hi = min(p, key_hi - 1);
-      // tree: bits [kb - start, kb - start + 64) of the row's mask (key kb + t is bit t)
-      uint64_t tbits = 0;
-      if (TREE) {
-        const int j0 = kb - tstart;
-        if (R.qval[qt] && j0 > -64 && j0 < tv.n) {
-          const int wq = j0 >> 6, sh = j0 & 63;  // floor division (j0 may be negative)
-          const uint64_t* mrow = tv.mask + (size_t)R.qnode[qt] * tv.words;
-          const uint64_t w0 = wq >= 0 ? mrow[wq] : 0ull;
-          const uint64_t w1 = wq + 1 < tv.words ? mrow[wq + 1] : 0ull;
-          tbits = sh == 0 ? w0 : (w0 >> sh) | (w1 << (64 - sh));
-        }
-      }
-#pragma unroll
-      for (int kt = 0; kt < 4; ++kt)
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-          const int key = kb + tile_key(kt, 4 * g + v);
-          bool ok;
-          if (TREE) {
-            if (key < tstart)
-              ok = key >= lo && key < key_hi;  // committed prefix (window on positions)
-            else  // tree slot: the mask (its window already applied for sliding layers)
-              ok = key >= key_lo && key < key_hi && ((tbits >> tile_key(kt, 4 * g + v)) & 1ull);
-            ok = ok && R.qval[qt];
-          } else {
-            ok = R.qval[qt] && key >= lo && key <= hi;
-          }
-          s[kt][v] = ok ? s[kt][v] : -INFINITY;
-          bmax = fmaxf(bmax, s[kt][v]);
-        }
-    }
-    bmax = max_lane_groups(bmax);
+    const float bmax = rows_mask_max<QT, TREE>(R, s, qt, kb, interior, key_lo, key_hi, window, tv);
     // (a fully masked row keeps m = -1e30: -1e30 + kMaxSlack rounds to -1e30 and -inf never exceeds it)
     const float m_blk = bmax * scale;
     const bool move = m_blk > R.m_run[qt] + kMaxSlack;
@@ -462,6 +482,188 @@ __device__ __forceinline__ void attn_item(const flyai_attn_item& it, int item_id
   }
 }
 
+// The same item by a workgroup of kCoopWaves waves, bit for bit attn_item's result.  What an item's 64-key
+// blocks must do in order is little -- the running max, and the accumulation of O and L -- so the rest is
+// divided: of each super-block of 4 NB blocks, wave w computes the scores and P of blocks w, w + 4, ..., and
+// accumulates dim tile w of O over all of them, in block order.  Between the two, the blocks' row maxima
+// (from which every wave derives the same running max) and then P pass through LDS; two barriers a
+// super-block.  K of the next super-block is requested when this one's scores are done, V after its PV.
+// For batches of few items: one wave an item is a chain of 16 blocks (load, QK, max, exp, PV) for a
+// 1024-key split, on a chip that is mostly idle: one token at KV 1500 (16 items) 16.0 -> 9.3 us, an 8-token
+// verify at KV 8000 (128 items) 24.7 -> 15.1 us.
+constexpr int kCoopWaves = 4;
+
+template <int QT, int NB>
+struct CoopShared {
+  float bm[kCoopWaves * NB][QT * 16];
+  uint4 p[kCoopWaves * NB][QT][2][64];
+};
+
+template <int QT, bool TREE, int NB>
+__device__ __forceinline__ void attn_item_coop(const flyai_attn_item& it, int item_idx,
+                                               const uint16_t* __restrict__ q,
+                                               const uint16_t* __restrict__ k_pool,
+                                               const uint16_t* __restrict__ v_pool,
+                                               const int64_t* __restrict__ kv_base,
+                                               const int32_t* __restrict__ kv_cap, int window, int Hq,
+                                               float* __restrict__ partials,
+                                               const flyai_attn_group* __restrict__ groups, int n_groups,
+                                               const float* __restrict__ sinks, uint16_t* __restrict__ out,
+                                               const TreeView& tv, CoopShared<QT, NB>& sh) {
+  constexpr int SB = kCoopWaves * NB;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int n = lane & 15, g = lane >> 4;
+  const float scale = 0.125f * kLog2e;
+  const bf16x8_t ones = as_bf16x8(make_uint4(0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u));
+  const bool single = it.group >= 0 && it.group < n_groups && groups[it.group].n_splits == 1;
+  const int cap = kv_cap[it.seq];
+  const int64_t base = kv_base[it.seq] + (int64_t)it.kv_head * cap * 64;
+  const uint16_t* K = k_pool + base;
+  const uint16_t* Vt = v_pool + base + wave * 512 + lane * 8;  // this wave's dim tile
+  const int kb_first = it.key_lo & ~63;
+  const int n_blk = (it.key_hi - kb_first + 63) >> 6, last = n_blk - 1;
+
+  uint4 kc[NB][4][2], vv[SB][2];
+  // block b of the item; past its last one, the last again (never computed on)
+  auto load_k = [&](int sb) __attribute__((always_inline)) {
+#pragma unroll
+    for (int j = 0; j < NB; ++j) load_k_tile(kc[j], K, kb_first + 64 * min(sb * SB + j * kCoopWaves + wave, last), lane);
+  };
+  auto load_v = [&](int sb) __attribute__((always_inline)) {
+#pragma unroll
+    for (int b = 0; b < SB; ++b) {
+      const uint16_t* blk = Vt + (size_t)(kb_first + 64 * min(sb * SB + b, last)) * 64;
+      vv[b][0] = ld_kv(blk);
+      vv[b][1] = ld_kv(blk + 2048);
+    }
+  };
+  load_k(0);
+  load_v(0);
+  QRows<QT> R;
+  rows_init<QT, TREE>(R, q, it.tok, it.ntok, it.pos0, it.kv_head, Hq, tv);
+  int pos_last, int_hi;
+  if (TREE) {
+    int dmax = 0;
+    for (int i = 0; i < it.ntok; ++i) dmax = max(dmax, tv.depth[it.tok + i]);
+    pos_last = tv.start + dmax;
+    int_hi = min(it.key_hi - 1, tv.start - 1);
+  } else {
+    pos_last = it.pos0 + it.ntok - 1;
+    int_hi = min(it.key_hi - 1, it.pos0);
+  }
+  const int int_lo = max(it.key_lo, window > 0 ? pos_last - window + 1 : 0);
+
+  auto step = [&](int sb, auto more) __attribute__((always_inline)) {
+    f32x4_t s[NB][QT][4];
+#pragma unroll
+    for (int j = 0; j < NB; ++j) {
+      const int blk = j * kCoopWaves + wave, kb = kb_first + 64 * (sb * SB + blk);
+      const bool interior = kb >= int_lo && kb + 63 <= int_hi;
+#pragma unroll
+      for (int qt = 0; qt < QT; ++qt) {
+#pragma unroll
+        for (int kt = 0; kt < 4; ++kt) {
+          s[j][qt][kt] = mfma16x16x32(as_bf16x8(kc[j][kt][0]), R.qf[qt][0], f32x4_t{0.f, 0.f, 0.f, 0.f});
+          s[j][qt][kt] = mfma16x16x32(as_bf16x8(kc[j][kt][1]), R.qf[qt][1], s[j][qt][kt]);
+        }
+        const float bmax = rows_mask_max<QT, TREE>(R, s[j][qt], qt, kb, interior, it.key_lo, it.key_hi, window, tv);
+        if (g == 0) sh.bm[blk][16 * qt + n] = bmax;
+      }
+    }
+    if constexpr (decltype(more)::value) load_k(sb + 1);
+    lds_barrier();
+    // the running max over the super-block's blocks, in order (as rows_block moves it)
+    float alpha[SB][QT], m_own[NB][QT];
+#pragma unroll
+    for (int b = 0; b < SB; ++b)
+#pragma unroll
+      for (int qt = 0; qt < QT; ++qt) {
+        const float m_blk = sh.bm[b][16 * qt + n] * scale;  // (a block past the last is not used)
+        const bool move = sb * SB + b < n_blk && m_blk > R.m_run[qt] + kMaxSlack;
+        const float m_new = move ? m_blk : R.m_run[qt];
+        alpha[b][qt] = R.m_run[qt] - m_new;
+        R.m_run[qt] = m_new;
+        if ((b % kCoopWaves) == wave) m_own[b / kCoopWaves][qt] = m_new;
+      }
+#pragma unroll
+    for (int j = 0; j < NB; ++j)
+#pragma unroll
+      for (int qt = 0; qt < QT; ++qt) {
+        const float neg_m = -m_own[j][qt];
+        bf16x8_t pt[2];
+#pragma unroll
+        for (int kt = 0; kt < 4; ++kt)
+#pragma unroll
+          for (int v = 0; v < 4; ++v)
+            pt[kt >> 1][(kt & 1) * 4 + v] = (__bf16)__builtin_amdgcn_exp2f(fmaf(s[j][qt][kt][v], scale, neg_m));
+        sh.p[j * kCoopWaves + wave][qt][0][lane] = __builtin_bit_cast(uint4, pt[0]);
+        sh.p[j * kCoopWaves + wave][qt][1][lane] = __builtin_bit_cast(uint4, pt[1]);
+      }
+    lds_barrier();
+#pragma unroll
+    for (int b = 0; b < SB; ++b) {
+      const int kb = kb_first + 64 * (sb * SB + b);
+      if (kb >= it.key_hi) break;  // uniform
+      uint4 v0 = vv[b][0], v1 = vv[b][1];
+      if (kb + 64 > it.key_hi) {
+        v0 = mask_keys(v0, kb + 8 * g, INT_MIN, it.key_hi);
+        v1 = mask_keys(v1, kb + 32 + 8 * g, INT_MIN, it.key_hi);
+      }
+#pragma unroll
+      for (int qt = 0; qt < QT; ++qt) {
+        if (__ballot(alpha[b][qt] != 0.f)) {
+          const float a = __builtin_amdgcn_exp2f(alpha[b][qt]);
+          R.L[qt] *= a;
+          R.O[qt][0] *= a;
+        }
+        const bf16x8_t p0 = as_bf16x8(sh.p[b][qt][0][lane]), p1 = as_bf16x8(sh.p[b][qt][1][lane]);
+        R.L[qt] = mfma16x16x32(ones, p0, R.L[qt]);
+        R.L[qt] = mfma16x16x32(ones, p1, R.L[qt]);
+        R.O[qt][0] = mfma16x16x32(as_bf16x8(v0), p0, R.O[qt][0]);
+        R.O[qt][0] = mfma16x16x32(as_bf16x8(v1), p1, R.O[qt][0]);
+      }
+    }
+    if constexpr (decltype(more)::value) load_v(sb + 1);
+  };
+  const int n_sb = (n_blk + SB - 1) / SB;
+  for (int sb = 0; sb + 1 < n_sb; ++sb) step(sb, std::true_type{});
+  step(n_sb - 1, std::false_type{});
+
+  // as attn_item's end, for dim tile `wave`
+  const int dt = wave;
+#pragma unroll
+  for (int qt = 0; qt < QT; ++qt) {
+    const float l = R.L[qt][0];
+    const int rq = 16 * qt + n;
+    if (!R.qval[qt]) continue;
+    if (single) {
+      const int h = it.kv_head * 8 + (rq & 7);
+      const float sink = sinks[h] * kLog2e;
+      const float M = fmaxf(sink, R.m_run[qt]);
+      float L = exp2f(sink - M);
+      const float wgt = exp2f(R.m_run[qt] - M);
+      L += l * wgt;
+      const float inv = 1.0f / L;
+      uint16_t* o = out + ((size_t)(it.tok + (rq >> 3)) * Hq + h) * 64;
+      float a[4];
+#pragma unroll
+      for (int v = 0; v < 4; ++v) a[v] = 0.f + R.O[qt][0][v] * wgt;
+      const uint32_t lo = (uint32_t)f2bf(a[0] * inv) | ((uint32_t)f2bf(a[1] * inv) << 16);
+      const uint32_t hi = (uint32_t)f2bf(a[2] * inv) | ((uint32_t)f2bf(a[3] * inv) << 16);
+      *reinterpret_cast<uint2*>(o + 16 * dt + 4 * g) = make_uint2(lo, hi);
+      continue;
+    }
+    float* rec = partials + ((size_t)item_idx * kAttnRows + rq) * kPartFloats;
+    if (g == 0 && dt == 0) {
+      rec[0] = R.m_run[qt];
+      rec[1] = l;
+    }
+#pragma unroll
+    for (int v = 0; v < 4; ++v) rec[2 + 16 * dt + 4 * g + v] = R.O[qt][0][v];
+  }
+}
+
 // One launch for every item; the body is chosen per item (uniform across the wave).
 __global__ __launch_bounds__(64, 2) void attn_partial_kernel(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ k_pool,
@@ -491,19 +693,79 @@ __global__ __launch_bounds__(64, 1) void attn_tree_kernel(
     const flyai_attn_group* __restrict__ groups, int n_groups, const float* __restrict__ sinks,
     uint16_t* __restrict__ out, const flyai_attn_tree* __restrict__ tree) {
   const flyai_attn_item it = items[blockIdx.x];
-  const char* tb = reinterpret_cast<const char*>(tree);
-  TreeView tv;
-  tv.start = tree->start;
-  tv.n = tree->n_nodes;
-  tv.words = tree->words;
-  tv.depth = reinterpret_cast<const int32_t*>(tb + tree->depth_off);
-  tv.mask = reinterpret_cast<const uint64_t*>(tb + tree->mask_off[window > 0 ? 1 : 0]);
+  const TreeView tv = tree_view(tree, window);
   if (it.ntok <= 2)
     attn_item<1, true>(it, blockIdx.x, q, k_pool, v_pool, kv_base, kv_cap, window, Hq, partials, groups, n_groups, sinks, out,
                        tv);
   else
     attn_item<2, true>(it, blockIdx.x, q, k_pool, v_pool, kv_base, kv_cap, window, Hq, partials, groups, n_groups, sinks, out,
                        tv);
+}
+
+// Blocks a wave of a super-block, for items of one and of two row tiles (two spill with two row tiles), and
+// the most blocks an item may have to be left to one wave, which needs no barrier: 32 windowed
+// single-token rows (3 blocks) 7.0 us by one wave, 7.6 by four; 8 windowed 4-token rows 7.8 and 6.8 us.
+constexpr int kCoopNB1 = 2, kCoopNB2 = 1;
+constexpr int kSoloBlocks1 = 3, kSoloBlocks2 = 1;
+
+union CoopAny {
+  CoopShared<1, kCoopNB1> one;
+  CoopShared<2, kCoopNB2> two;
+};
+
+template <int QT, bool TREE, int NB, int SOLO>
+__device__ __forceinline__ void attn_item_any(const flyai_attn_item& it, const uint16_t* __restrict__ q,
+                                              const uint16_t* __restrict__ k_pool,
+                                              const uint16_t* __restrict__ v_pool,
+                                              const int64_t* __restrict__ kv_base,
+                                              const int32_t* __restrict__ kv_cap, int window, int Hq,
+                                              float* __restrict__ partials,
+                                              const flyai_attn_group* __restrict__ groups, int n_groups,
+                                              const float* __restrict__ sinks, uint16_t* __restrict__ out,
+                                              const TreeView& tv, CoopShared<QT, NB>& sh) {
+  if (it.key_hi - (it.key_lo & ~63) > 64 * SOLO)
+    attn_item_coop<QT, TREE, NB>(it, blockIdx.x, q, k_pool, v_pool, kv_base, kv_cap, window, Hq, partials, groups,
+                                 n_groups, sinks, out, tv, sh);
+  else if (threadIdx.x < 64)
+    attn_item<QT, TREE>(it, blockIdx.x, q, k_pool, v_pool, kv_base, kv_cap, window, Hq, partials, groups, n_groups,
+                        sinks, out, tv);
+}
+
+// attn_partial_kernel and attn_tree_kernel with a workgroup of kCoopWaves waves an item
+__global__ __launch_bounds__(64 * kCoopWaves, 2) void attn_coop_kernel(
+    const uint16_t* __restrict__ q, const uint16_t* __restrict__ k_pool,
+    const uint16_t* __restrict__ v_pool, const int64_t* __restrict__ kv_base,
+    const int32_t* __restrict__ kv_cap, int window, int Hq,
+    const flyai_attn_item* __restrict__ items, const int32_t* __restrict__ n_live,
+    float* __restrict__ partials, const flyai_attn_group* __restrict__ groups, int n_groups,
+    const float* __restrict__ sinks, uint16_t* __restrict__ out) {
+  __shared__ CoopAny sh;
+  if (n_live && (int)blockIdx.x >= *n_live) return;  // as in attn_partial_kernel
+  const flyai_attn_item it = items[blockIdx.x];
+  if (it.ntok <= 2)
+    attn_item_any<1, false, kCoopNB1, kSoloBlocks1>(it, q, k_pool, v_pool, kv_base, kv_cap, window, Hq, partials, groups,
+                                                    n_groups, sinks, out, TreeView{}, sh.one);
+  else
+    attn_item_any<2, false, kCoopNB2, kSoloBlocks2>(it, q, k_pool, v_pool, kv_base, kv_cap, window, Hq, partials, groups,
+                                                    n_groups, sinks, out, TreeView{}, sh.two);
+}
+
+__global__ __launch_bounds__(64 * kCoopWaves, 1) void attn_tree_coop_kernel(
+    const uint16_t* __restrict__ q, const uint16_t* __restrict__ k_pool,
+    const uint16_t* __restrict__ v_pool, const int64_t* __restrict__ kv_base,
+    const int32_t* __restrict__ kv_cap, int window, int Hq,
+    const flyai_attn_item* __restrict__ items, float* __restrict__ partials,
+    const flyai_attn_group* __restrict__ groups, int n_groups, const float* __restrict__ sinks,
+    uint16_t* __restrict__ out, const flyai_attn_tree* __restrict__ tree) {
+  __shared__ CoopAny sh;
+  const flyai_attn_item it = items[blockIdx.x];
+  const TreeView tv = tree_view(tree, window);
+  if (it.ntok <= 2)
+    attn_item_any<1, true, kCoopNB1, kSoloBlocks1>(it, q, k_pool, v_pool, kv_base, kv_cap, window, Hq, partials, groups,
+                                                   n_groups, sinks, out, tv, sh.one);
+  else
+    attn_item_any<2, true, kCoopNB2, kSoloBlocks2>(it, q, k_pool, v_pool, kv_base, kv_cap, window, Hq, partials, groups,
+                                                   n_groups, sinks, out, tv, sh.two);
 }
 
 // ---- chunked-prefill rows -------------------------------------------------------------------------
@@ -765,6 +1027,12 @@ __global__ __launch_bounds__(256) void attn_merge_kernel(const float* __restrict
   *reinterpret_cast<uint4*>(o) = make_uint4(wv[0], wv[1], wv[2], wv[3]);
 }
 
+// Up to this many items a workgroup of four waves takes each; past it the chip is full with one wave an item
+// and the barriers only cost.  One wave / four waves an item, items of up to 16 blocks: 16 items 16.0 /
+// 9.3 us, 128 24.7 / 15.1, 248 25.2 / 16.7, 384 27.4 / 21.2, 544 34.1 / 30.3, 880 39.8 / 41.1,
+// 1264 48.8 / 52.7.
+constexpr int kCoopItems = 640;
+
 // n_items / n_groups size the grids; counts (nullable) holds this step's live item and group
 // counts on the device, for launches sized by a plan capacity (graph replay)
 int launch_attn(const uint16_t* q, const uint16_t* k_pool, const uint16_t* v_pool,
@@ -774,9 +1042,16 @@ int launch_attn(const uint16_t* q, const uint16_t* k_pool, const uint16_t* v_poo
                 uint16_t* out, const flyai_attn_tree* tree, bool merge, hipStream_t s) {
   if (n_items == 0) return FLYAI_OK;
   (void)n_small;  // the plan's two ranges share one launch
-  if (tree)  // launched directly with exact counts (never from a graph)
+  const bool coop = n_items <= kCoopItems;
+  if (tree && coop)  // a tree is launched directly with exact counts (never from a graph)
+    hipLaunchKernelGGL(attn_tree_coop_kernel, dim3(n_items), dim3(64 * kCoopWaves), 0, s, q, k_pool, v_pool, kv_base,
+                       kv_cap, window, Hq, items, partials, groups, n_groups, sinks, out, tree);
+  else if (tree)
     hipLaunchKernelGGL(attn_tree_kernel, dim3(n_items), dim3(64), 0, s, q, k_pool, v_pool, kv_base, kv_cap, window,
                        Hq, items, partials, groups, n_groups, sinks, out, tree);
+  else if (coop)
+    hipLaunchKernelGGL(attn_coop_kernel, dim3(n_items), dim3(64 * kCoopWaves), 0, s, q, k_pool, v_pool, kv_base,
+                       kv_cap, window, Hq, items, counts, partials, groups, n_groups, sinks, out);
   else
     hipLaunchKernelGGL(attn_partial_kernel, dim3(n_items), dim3(64), 0, s, q, k_pool, v_pool, kv_base,
                        kv_cap, window, Hq, items, counts, partials, groups, n_groups, sinks, out);

@@ -416,6 +416,47 @@ def test_attention_prefill_items_vs_oracle(window):
     assert mar0 < 1e-2 and cos0 > 0.99999
 
 
+@pytest.mark.parametrize("window,split", [(0, 1024), (0, 192), (128, 1024)])
+def test_attention_few_items_equal_many_items_bit_exact(window, split):
+    """A launch of few items gives each one four waves, a launch of many one wave each: every sequence
+    alone (few items) equals the same sequence among the others (many items), bit for bit.  Lengths at the
+    edges of blocks, of a super-block (256 and 512 keys) and of a split; 1 to 8 query tokens; logits large
+    enough to move the running max often; NaN in the unwritten slots."""
+    from flyai_amd import ops
+    Hq, Hkv, D = 64, 8, 64
+    ends = [1, 2, 63, 64, 65, 129, 255, 256, 257, 512, 513, 1000, 1023, 1024, 1025, 2047, 2300]
+    seqs = [(q, max(0, e - q)) for e in ends for q in (1, 2, 3, 8)]
+    q_lens, starts = [q for q, _ in seqs], [s for _, s in seqs]
+    cap = 2432
+    S, T, slab = len(seqs), sum(q_lens), Hkv * cap * D
+    kp = torch.full((S * slab,), float("nan"), device=DEV, dtype=torch.bfloat16)
+    vp = torch.full((S * slab,), float("nan"), device=DEV, dtype=torch.bfloat16)
+    for b, (ql, st) in enumerate(seqs):
+        pos = torch.arange(st + ql, device=DEV)
+        kvlayout.scatter(kp[b * slab:(b + 1) * slab], Hkv, cap, "k",
+                         4 * torch.randn(Hkv, st + ql, D, device=DEV, generator=_gen(300 + b)), pos)
+        kvlayout.scatter(vp[b * slab:(b + 1) * slab], Hkv, cap, "v",
+                         torch.randn(Hkv, st + ql, D, device=DEV, generator=_gen(500 + b)), pos)
+    q = (4 * torch.randn(T, Hq, D, device=DEV, generator=_gen(54))).to(torch.bfloat16)
+    sinks = torch.randn(Hq, device=DEV, generator=_gen(55)).to(torch.bfloat16).float()
+
+    def run(sel, rows):
+        base = torch.tensor([b * slab for b in sel], dtype=torch.int64, device=DEV)
+        capt = torch.tensor([cap] * len(sel), dtype=torch.int32, device=DEV)
+        items, groups, n_small = ops.attn_plan([q_lens[b] for b in sel], [starts[b] for b in sel], Hkv, window, split)
+        return ops.attn_ragged(rows.contiguous(), kp, vp, base, capt, sinks, window, items, groups, n_small, Hkv), len(items)
+
+    many, n = run(range(S), q)
+    assert n > 640
+    t = 0
+    for b, ql in enumerate(q_lens):
+        few, n = run([b], q[t:t + ql])
+        assert n <= 512
+        assert torch.equal(few.view(torch.int16), many[t:t + ql].view(torch.int16)), (q_lens[b], starts[b])
+        t += ql
+    assert torch.isfinite(many.float()).all()
+
+
 def test_attention_ignores_unwritten_nan_slots():
     """Keys/values past each sequence's length (and before its window) are never read into the
     result even when they hold NaN: the kernel masks scores and zeroes out-of-range values."""
