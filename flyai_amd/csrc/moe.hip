@@ -356,7 +356,7 @@ constexpr int kDepthDown = 8;
 // 4-way unrolled group loop is straight-line; a block's outputs are written after its last group.
 // Loads are unconditional with clamped addresses: rows past the group read row 0 and are never
 // stored; weight lanes past a row's last block (and the padding groups) are zeroed before
-// conversion, their activation slots read the row's first group (finite values); tiles past N
+// conversion, their activation slots read zeros; tiles past N
 // load a clamped tile whose codes are zeroed before conversion (MFMAs on zero operands draw less
 // power: down at 128 experts x 65 rows 194-195 -> 192 us) and are never stored; the 3 groups issued
 // past the chunk's end read clamped addresses and are never computed on.
@@ -383,11 +383,11 @@ __device__ __forceinline__ int act_swz(int r) {
 }
 
 // Work units of the dense GEMMs: every group of at least min_rows rows is cut into passes of
-// kGemmRows rows, the passes are numbered expert by expert, and unit u is weight-block chunk
+// ROWS rows, the passes are numbered expert by expert, and unit u is weight-block chunk
 // u % chunks_per_e of pass u / chunks_per_e.  A group of many rows (a hot expert) so spreads its
 // passes over workgroups instead of running them one after another in each of its workgroups.  Every
 // workgroup derives the numbering from offsets[0..E] (an exclusive scan in LDS); the grid is sized for
-// the most passes any routing can give, sum_e ceil(n_e / kGemmRows) <= rows_total / kGemmRows + E, and
+// the most passes any routing can give, sum_e ceil(n_e / ROWS) <= rows_total / ROWS + E, and
 // units past the last pass exit.
 
 struct DenseUnit {
@@ -398,6 +398,7 @@ struct DenseUnit {
 // live units are spread over the 8 XCDs, consecutive ones on one XCD (workgroups are dealt to the XCDs
 // round-robin by index), so that an XCD's L2 serves a pass's activation rows to all its chunks and
 // the units past the live count, which exit, do not leave XCDs idle.
+template <int ROWS>
 __device__ __forceinline__ bool dense_unit(const int32_t* __restrict__ offsets, int E, int min_rows,
                                            int chunks_per_e, int* pre, DenseUnit& u, int& unit) {
   const int tid = threadIdx.x;
@@ -407,7 +408,7 @@ __device__ __forceinline__ bool dense_unit(const int32_t* __restrict__ offsets, 
     for (int j = 0; j < 4; ++j) {
       const int e = 4 * tid + j;
       const int n = e < E ? offsets[e + 1] - offsets[e] : 0;
-      v[j] = (n > 0 && n >= min_rows) ? (n + kGemmRows - 1) / kGemmRows : 0;
+      v[j] = (n > 0 && n >= min_rows) ? (n + ROWS - 1) / ROWS : 0;
       sum += v[j];
     }
     int incl = sum;
@@ -441,8 +442,8 @@ __device__ __forceinline__ bool dense_unit(const int32_t* __restrict__ offsets, 
   u.e = e;
   u.row_lo = offsets[e];
   u.n_e = offsets[e + 1] - u.row_lo;
-  u.m0 = (p - pre[e]) * kGemmRows;
-  u.rows = min(kGemmRows, u.n_e - u.m0);
+  u.m0 = (p - pre[e]) * ROWS;
+  u.rows = min(ROWS, u.n_e - u.m0);
   return true;
 }
 
@@ -464,9 +465,10 @@ struct GemmCtx {
 // global load in the loop, and waiting for it (vector-memory counts complete in issue order) would
 // drain the groups prefetched behind it.
 constexpr int kGemmBiasBlocks = 32;
+template <int BIAS>
 __device__ __forceinline__ void stage_chunk_bias(const float* __restrict__ bias, int e, int N, int nb0, int nbn,
-                                                 float (&bias_s)[kGemmBiasBlocks * 256]) {
-  constexpr int kPer = kGemmBiasBlocks * 256 / 512;
+                                                 float (&bias_s)[BIAS]) {
+  constexpr int kPer = BIAS / 512;
   float v[kPer];
 #pragma unroll
   for (int j = 0; j < kPer; ++j) {
@@ -478,11 +480,14 @@ __device__ __forceinline__ void stage_chunk_bias(const float* __restrict__ bias,
   for (int j = 0; j < kPer; ++j) bias_s[threadIdx.x + j * 512] = v[j];
 }
 
+// what the activation loads past a row's end read
+__device__ __align__(16) uint16_t g_zero_chunk[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+
 // One pass over MT row tiles (16*MT rows from m0) and every block of the chunk.
-template <bool GATE_UP, int MT>
-__device__ __forceinline__ void gemm_pass(const GemmCtx& c, char (&st0)[kGemmStage], char (&st1)[kGemmStage],
-                                          char (&st2)[kGemmStage], char (&st3)[kGemmStage],
-                                          float (&bias_s)[kGemmBiasBlocks * 256], int m0, int rows) {
+template <bool GATE_UP, int MT, int STAGE, int BIAS>
+__device__ __forceinline__ void gemm_pass(const GemmCtx& c, char (&st0)[STAGE], char (&st1)[STAGE],
+                                          char (&st2)[STAGE], char (&st3)[STAGE],
+                                          float (&bias_s)[BIAS], int m0, int rows) {
   typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
   typedef __attribute__((address_space(3))) void* lds_ptr;
   static_assert(MT >= 1 && MT <= 6, "row tiles per pass");
@@ -532,12 +537,12 @@ __device__ __forceinline__ void gemm_pass(const GemmCtx& c, char (&st0)[kGemmSta
     for (int n = 0; n < 2; ++n)
       __builtin_amdgcn_global_load_lds((const void*)(c.sbase + ((size_t)tile_of(nb, n) * gm.KG4 + min(kg / 4, gm.KG4 - 1)) * 256),
                                        (lds_ptr)(stage + ABYTES + (2 * wave + n) * 256), 4, 0, 0);
-    // a chunk past the row's last block (or of a padding group) reads the row's first group instead:
-    // in bounds and finite, and multiplied only by zeroed weights
+    // a chunk past the row's last block (or of a padding group) reads zeros: its weights are zeroed too, but
+    // a row's own first group in its place would turn an infinity there into a NaN
 #pragma unroll
     for (int J = 0; J < MD; ++J) {
-      const int col = 4 * kg + ablk[J] < gm.G ? kg * 128 : 0;
-      __builtin_amdgcn_global_load_lds((const void*)(arow[J] + col), (lds_ptr)(stage + (J * 8 + wave) * 1024), 16, 0, 0);
+      const uint16_t* src = 4 * kg + ablk[J] < gm.G ? arow[J] + kg * 128 : g_zero_chunk;
+      __builtin_amdgcn_global_load_lds((const void*)src, (lds_ptr)(stage + (J * 8 + wave) * 1024), 16, 0, 0);
     }
     if (++i_kg == KGP) {
       i_kg = 0;
@@ -705,24 +710,13 @@ __device__ __forceinline__ void gemm_pass(const GemmCtx& c, char (&st0)[kGemmSta
   __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));  // the loads past the chunk's end have landed
 }
 
-template <bool GATE_UP>
-__global__ __launch_bounds__(512) void moe_mxfp4_gemm_kernel(
-    const uint16_t* __restrict__ act, const int32_t* __restrict__ perm,
-    const int32_t* __restrict__ offsets, int k_top, const uint8_t* __restrict__ packed,
-    const float* __restrict__ bias, int E, int N, int K, int min_rows, int chunk, void* __restrict__ out) {
-  __shared__ __align__(16) char st0[kGemmStage];
-  __shared__ __align__(16) char st1[kGemmStage];
-  __shared__ __align__(16) char st2[kGemmStage];
-  __shared__ __align__(16) char st3[kGemmStage];
+// The unit's context for a workgroup of 8 waves; chunks_per_e chunks of `chunk` weight blocks an expert.
+__device__ __forceinline__ GemmCtx gemm_ctx(const MxGeom& gm, const DenseUnit& du, int unit, int blocks_per_e,
+                                            int chunks_per_e, int chunk, const uint16_t* act, const int32_t* perm,
+                                            int k_top, const uint8_t* packed, const float* bias, int N, int K,
+                                            void* out) {
   GemmCtx c;
-  c.gm = mx_geom(E, N, K);
-  const int blocks_per_e = (c.gm.NT + kGemmTiles - 1) / kGemmTiles;
-  const int chunks_per_e = (blocks_per_e + chunk - 1) / chunk;
-  __shared__ int pass_pre[257];
-  __shared__ float bias_s[kGemmBiasBlocks * 256];
-  DenseUnit du;
-  int unit = 0;
-  if (!dense_unit(offsets, E, min_rows, chunks_per_e, pass_pre, du, unit)) return;
+  c.gm = gm;
   c.e = du.e;
   c.nb0 = (unit % chunks_per_e) * chunk;
   c.nbn = min(chunk, blocks_per_e - c.nb0);  // weight blocks in this chunk
@@ -739,15 +733,71 @@ __global__ __launch_bounds__(512) void moe_mxfp4_gemm_kernel(
   c.wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   c.r = c.lane & 15;
   c.g = c.lane >> 4;
-  c.tile_bytes = (size_t)c.gm.G * 256;
-  c.wbase = packed + (size_t)c.e * c.gm.NT * c.tile_bytes + c.lane * 16;
-  c.sbase = packed + c.gm.data_bytes + (size_t)c.e * c.gm.NT * c.gm.KG4 * 256 + c.lane * 4;
+  c.tile_bytes = (size_t)gm.G * 256;
+  c.wbase = packed + (size_t)c.e * gm.NT * c.tile_bytes + c.lane * 16;
+  c.sbase = packed + gm.data_bytes + (size_t)c.e * gm.NT * gm.KG4 * 256 + c.lane * 4;
+  return c;
+}
+
+template <bool GATE_UP>
+__global__ __launch_bounds__(512) void moe_mxfp4_gemm_kernel(
+    const uint16_t* __restrict__ act, const int32_t* __restrict__ perm,
+    const int32_t* __restrict__ offsets, int k_top, const uint8_t* __restrict__ packed,
+    const float* __restrict__ bias, int E, int N, int K, int min_rows, int chunk, void* __restrict__ out) {
+  __shared__ __align__(16) char st0[kGemmStage];
+  __shared__ __align__(16) char st1[kGemmStage];
+  __shared__ __align__(16) char st2[kGemmStage];
+  __shared__ __align__(16) char st3[kGemmStage];
+  __shared__ int pass_pre[257];
+  __shared__ float bias_s[kGemmBiasBlocks * 256];
+  const MxGeom gm = mx_geom(E, N, K);
+  const int blocks_per_e = (gm.NT + kGemmTiles - 1) / kGemmTiles;
+  const int chunks_per_e = (blocks_per_e + chunk - 1) / chunk;
+  DenseUnit du;
+  int unit = 0;
+  if (!dense_unit<kGemmRows>(offsets, E, min_rows, chunks_per_e, pass_pre, du, unit)) return;
+  const GemmCtx c = gemm_ctx(gm, du, unit, blocks_per_e, chunks_per_e, chunk, act, perm, k_top, packed, bias, N, K, out);
   // this unit's pass of up to 96 rows, as the fewest 16-row tiles that hold them (at least 2)
   if (du.rows > 80) gemm_pass<GATE_UP, 6>(c, st0, st1, st2, st3, bias_s, du.m0, du.rows);
   else if (du.rows > 64) gemm_pass<GATE_UP, 5>(c, st0, st1, st2, st3, bias_s, du.m0, du.rows);
   else if (du.rows > 48) gemm_pass<GATE_UP, 4>(c, st0, st1, st2, st3, bias_s, du.m0, du.rows);
   else if (du.rows > 32) gemm_pass<GATE_UP, 3>(c, st0, st1, st2, st3, bias_s, du.m0, du.rows);
   else gemm_pass<GATE_UP, 2>(c, st0, st1, st2, st3, bias_s, du.m0, du.rows);
+}
+
+// ---- batches of medium groups -----------------------------------------------------------------------
+// Between the row-pass kernel, whose weight stream is read once per 8 rows, and the 96-row GEMM, whose one
+// workgroup a CU holds too few loads in flight to stream the weights of groups this small: the GEMM's pass
+// over at most two row tiles (32 rows), whose stages and registers are small enough for two workgroups of
+// 8 waves a CU (57 KB of LDS, 107-114 registers).  It serves every group of the batch, larger ones in
+// passes of 32 rows.  Same MFMA, K-to-lane mapping and order per output element as the other two, so the
+// same bits.  Rows an expert on average, 128 experts, H = I = 2880, before (row-pass and GEMM launches) and
+// with this kernel, gate_up / down: 6.3 rows 221 / 127 -> 213 / 117 us, 10.4 293 / 163 -> 225 / 125,
+// 16 279 / 161 -> 243 / 132.  What bounds it is the weight stream (5.0-5.4 TB/s).
+constexpr int kMidRows = 32;
+constexpr int kMidChunk = 3;  // weight blocks a unit: 2 to 6 within 3 % for gate_up; down 117 us with 3, 122-136 with 1, 2, 4, 6
+
+template <bool GATE_UP>
+__global__ __launch_bounds__(512, 4) void moe_mxfp4_mid_kernel(
+    const uint16_t* __restrict__ act, const int32_t* __restrict__ perm,
+    const int32_t* __restrict__ offsets, int k_top, const uint8_t* __restrict__ packed,
+    const float* __restrict__ bias, int E, int N, int K, int chunk, void* __restrict__ out) {
+  constexpr int kStage = kMidRows * 256 + kGemmTiles * 256;
+  __shared__ __align__(16) char st0[kStage];
+  __shared__ __align__(16) char st1[kStage];
+  __shared__ __align__(16) char st2[kStage];
+  __shared__ __align__(16) char st3[kStage];
+  __shared__ int pass_pre[257];
+  __shared__ float bias_s[4 * 256];  // at least kMidChunk blocks, in whole rounds of the 512 threads
+  const MxGeom gm = mx_geom(E, N, K);
+  const int blocks_per_e = (gm.NT + kGemmTiles - 1) / kGemmTiles;
+  const int chunks_per_e = (blocks_per_e + chunk - 1) / chunk;
+  DenseUnit du;
+  int unit = 0;
+  if (!dense_unit<kMidRows>(offsets, E, 1, chunks_per_e, pass_pre, du, unit)) return;
+  const GemmCtx c = gemm_ctx(gm, du, unit, blocks_per_e, chunks_per_e, chunk, act, perm, k_top, packed, bias, N, K, out);
+  if (du.rows > 16) gemm_pass<GATE_UP, 2>(c, st0, st1, st2, st3, bias_s, du.m0, du.rows);
+  else gemm_pass<GATE_UP, 1>(c, st0, st1, st2, st3, bias_s, du.m0, du.rows);
 }
 
 // ---- dense groups on the scaled MFMA: fp8 activations x MXFP4 weights -------------------------------
@@ -1084,7 +1134,7 @@ __global__ __launch_bounds__(512) void moe_mx_gemm_kernel(
   __shared__ float bias_s[kGemmBiasBlocks * 256];
   DenseUnit du;
   int unit = 0;
-  if (!dense_unit(offsets, E, min_rows, chunks_per_e, pass_pre, du, unit)) return;
+  if (!dense_unit<kGemmRows>(offsets, E, min_rows, chunks_per_e, pass_pre, du, unit)) return;
   c.e = du.e;
   c.nb0 = (unit % chunks_per_e) * chunk;
   c.nbn = min(chunk, blocks_per_e - c.nb0);
@@ -1146,12 +1196,36 @@ inline int gemm_grid(const MxGeom& gm, int E, int chunk, int rows_total) {
   return ((units + 7) / 8) * 8;
 }
 
+// launches the medium-group kernel; the chunk is kMidChunk weight blocks, or one where that leaves a CU without
+// its two workgroups
+template <bool GATE_UP>
+int launch_moe_mid(const uint16_t* act, const int32_t* perm, const int32_t* offsets, int k_top, const uint8_t* packed,
+                   const float* bias, int rows_total, int E, int N, int K, void* out, hipStream_t s) {
+  const MxGeom gm = mx_geom(E, N, K);
+  const int W = (gm.NT + kGemmTiles - 1) / kGemmTiles;
+  const int chunk = (int64_t)E * ceil_div(W, kMidChunk) >= 2LL * device_cus() ? kMidChunk : 1;
+  const int units = (E + ceil_div(rows_total, kMidRows)) * ceil_div(W, chunk);
+  hipLaunchKernelGGL((moe_mxfp4_mid_kernel<GATE_UP>), dim3((units + 7) / 8 * 8), dim3(512), 0, s, act, perm, offsets,
+                     k_top, packed, bias, E, N, K, chunk, out);
+  return check_launch(GATE_UP ? "moe_gate_up_mxfp4(mid)" : "moe_down_mxfp4(mid)");
+}
+
 // Groups of more than kDenseFrom rows take the dense kernel when the batch averages at least that
 // many rows per expert (otherwise the row-pass kernel serves every group: a rare large group costs
 // extra passes, not a launch of mostly idle workgroups).  Both kernels are correct for any count.
 constexpr int kDenseFrom = 8;
 
 inline bool use_dense(int rows_total, int E) { return (int64_t)rows_total >= (int64_t)kDenseFrom * E; }
+
+// Batches of kMidFrom to kMidTo rows per expert on average take the medium-group kernel alone.  gate_up + down,
+// 128 experts: at 4.7 rows the row-pass kernel takes 302 us and this one 328, at 6.3 348 and 331, at 8 409
+// and 346; at 16 the row-pass and GEMM launches together take 440 and this one 375, at 18 416 and 387; at
+// 22 the GEMM takes 434, and this one would run a second pass for most groups.
+constexpr int kMidFrom = 6, kMidTo = 18;
+
+inline bool use_mid(int rows_total, int E, int K) {
+  return K >= 128 && K <= 4064 && (int64_t)rows_total >= (int64_t)kMidFrom * E && (int64_t)rows_total < (int64_t)kMidTo * E;
+}
 
 // whether a batch of rows_total permuted rows gives any expert group to the dense kernels
 bool moe_batch_is_dense(int rows_total, int E, int K) { return use_dense(rows_total, E) && K >= 128; }
@@ -1160,6 +1234,7 @@ int launch_moe_gate_up(const uint16_t* x, const int32_t* perm, const int32_t* of
                        const uint8_t* w13, const float* b13, int T, int E, int H, int I, uint16_t* h,
                        hipStream_t s) {
   const MxGeom gm = mx_geom(E, 2 * I, H);
+  if (use_mid(T * k_top, E, H)) return launch_moe_mid<true>(x, perm, offsets, k_top, w13, b13, T * k_top, E, 2 * I, H, h, s);
   const bool dense = use_dense(T * k_top, E) && H >= 128;  // the tiled kernel reads 128-K groups
   if (H <= 4064) {
     const int wg_per_e = ceil_div(gm.NT, 4 * kNTWGateUp);
@@ -1182,6 +1257,7 @@ int launch_moe_gate_up(const uint16_t* x, const int32_t* perm, const int32_t* of
 int launch_moe_down(const uint16_t* h, const int32_t* offsets, const uint8_t* w2, const float* b2,
                     int rows_total, int E, int H, int I, float* y, hipStream_t s) {
   const MxGeom gm = mx_geom(E, H, I);
+  if (use_mid(rows_total, E, I)) return launch_moe_mid<false>(h, nullptr, offsets, 1, w2, b2, rows_total, E, H, I, y, s);
   const bool dense = use_dense(rows_total, E) && I >= 128;  // the tiled kernel reads 128-K groups
   if (I <= 4064) {
     const int wg_per_e = ceil_div(gm.NT, 4 * kNTWDown);

@@ -35,17 +35,31 @@ def _group(md):
 
 
 @pytest.fixture(scope="module")
-def gemm_asm(tmp_path_factory):
+def moe_asm(tmp_path_factory):
     out = tmp_path_factory.mktemp("asm") / "moe.s"
     flags = [f for f in B.FLAGS if f != "-fPIC"]
     r = subprocess.run([HIPCC, *flags, "-S", "--cuda-device-only", "-x", "hip",
                         os.path.join(B.CSRC, "moe.hip"), "-o", str(out)], capture_output=True, text=True)
     assert r.returncode == 0, r.stderr[-2000:]
-    text = out.read_text()
+    return out.read_text()
+
+
+def _bodies(text, kernel):
     bodies = {}
-    for name in re.findall(r"\n(_ZN5flyai21moe_mxfp4_gemm_kernel\w+):", text):
+    for name in re.findall(r"\n(_ZN5flyai\d+" + kernel + r"\w+):", text):
         i = text.index("\n" + name + ":")
         bodies[name] = text[i:text.index(".Lfunc_end", i)].split("\n")
+    return bodies
+
+
+@pytest.fixture(scope="module")
+def gemm_asm_mid(moe_asm):
+    return _bodies(moe_asm, "moe_mxfp4_mid_kernel")
+
+
+@pytest.fixture(scope="module")
+def gemm_asm(moe_asm):
+    bodies = _bodies(moe_asm, "moe_mxfp4_gemm_kernel")
     assert len(bodies) == 2, "expected the gate_up and down instantiations"
     return bodies
 
@@ -105,3 +119,19 @@ def test_prologue_issues_groups_in_order(gemm_asm):
                 assert not head - _group(md), f"{name} MD={md}: {ops}"
             checked += 1
         assert checked == 5, f"{name}: expected one prologue wait per row-tile count"
+
+
+def test_medium_kernel_groups(gemm_asm_mid):
+    """The medium-group kernel runs the same pass over one and two row tiles (MD = 1 for both)."""
+    assert len(gemm_asm_mid) == 2
+    for name, body in gemm_asm_mid.items():
+        loops = [n for n, l in enumerate(body) if "Inner Loop Header" in l]
+        assert len(loops) == 2, f"{name}: one group loop per row-tile count"
+        for lo in loops:
+            hi = next(n for n in range(lo, len(body)) if re.search(r"s_cbranch\w* \.LBB", body[n]))
+            waits = [n for n in range(lo, hi) if re.search(r"s_waitcnt vmcnt\(\d+\)", body[n])]
+            assert {int(re.search(r"vmcnt\((\d+)\)", body[w]).group(1)) for w in waits} == {10}
+            assert not any("scratch_" in body[n] for n in range(lo, hi)), f"{name}: spill code in a group loop"
+            bounds = waits + [hi]
+            for a, b in zip(bounds, bounds[1:]):
+                assert Counter(_ops(body[a:b])) == _group(1), f"{name}: group issue {_ops(body[a:b])}"

@@ -668,3 +668,35 @@ def test_dense_and_row_pass_experts_bit_identical():
             rb = torch.arange(ob[e], ob[e] + len(sel), device=DEV)
             assert torch.equal(h_a[ra], h_b[rb]), f"expert {e}, tokens {sel}: gate_up differs"
             assert torch.equal(y_a[ra], y_b[rb]), f"expert {e}, tokens {sel}: down differs"
+
+
+@pytest.mark.parametrize("H,I", [(2880, 2880), (128, 160), (544, 2048)])
+def test_medium_group_experts_bit_identical(H, I):
+    """A batch of 6 to 18 rows per expert on average runs the medium-group kernel; the same rows in batches
+    of at most 5 per expert run the row-pass kernel: h and y equal bit for bit.  Groups of 0 rows, of one
+    row tile and its neighbours, of two and their neighbours, and of more than a pass; K of whole and partial
+    128-K groups; fewer weight blocks than a chunk; rows holding an infinity (first and last group) and a NaN."""
+    from flyai_amd import ops
+    from flyai_amd.weights import GptOssShape, synthetic_moe
+    sizes = [1, 15, 0, 16, 17, 32, 33, 14]
+    E, T = len(sizes), sum(sizes)
+    assert 6 * E <= T < 18 * E
+    m = synthetic_moe(GptOssShape(hidden=H, intermediate=I, n_experts=E), _gen(61), DEV)
+    w13 = ops.mxfp4_repack(m["w13_blocks"], m["w13_scales"])
+    w2 = ops.mxfp4_repack(m["w2_blocks"], m["w2_scales"])
+    x = _rms_input(T, H, 62)
+    x[3, 5], x[40, H - 1], x[70, 1] = float("inf"), float("-inf"), float("nan")
+    ids = torch.cat([torch.full((n,), e) for e, n in enumerate(sizes)])[torch.randperm(T, generator=torch.Generator().manual_seed(3))]
+    ids = ids.to(torch.int32).to(DEV)[:, None].contiguous()
+
+    def run(rows):
+        _, off, perm, inv = ops.moe_permute(ids[rows].contiguous(), E)
+        h = ops.moe_gate_up(x[rows].contiguous(), perm, off, 1, w13, m["b13"], E, I)
+        return h[inv.long()], ops.moe_down(h, off, w2, m["b2"], E, H)[inv.long()]
+
+    h_all, y_all = run(torch.arange(T, device=DEV))
+    for t0 in range(0, T, 5 * E):
+        rows = torch.arange(t0, min(T, t0 + 5 * E), device=DEV)
+        h, y = run(rows)
+        assert torch.equal(h.view(torch.int16), h_all[rows].view(torch.int16)), "gate_up differs"
+        assert torch.equal(y.view(torch.int32), y_all[rows].view(torch.int32)), "down differs"
