@@ -214,7 +214,7 @@ inline int ceil_div(int a, int b) { return (a + b - 1) / b; }
 // entry behind it moves down one place (the last falls off) -- equal values keep the earlier (lower)
 // id ahead, the same list a strict-greater insertion at the end followed by bubbling past strictly
 // smaller values gives.  Every comparison is of the new entry (comparing a displaced entry again
-// would swap two equal values), and no comparison waits on another.  topk_insert_ordered: the same under (value desc, id asc).
+// would swap two equal values), and no comparison waits on another.
 template <int K>
 __device__ __forceinline__ void topk_insert_at(float (&sv)[K], int (&si)[K], float v, int id, const bool (&gt)[K]) {
   // gt[] is monotonic over the sorted list (false ... false, true ... true): the new entry goes to
@@ -235,14 +235,6 @@ __device__ __forceinline__ void topk_insert_strict(float (&sv)[K], int (&si)[K],
   bool gt[K];
 #pragma unroll
   for (int j = 0; j < K; ++j) gt[j] = v > sv[j];
-  topk_insert_at<K>(sv, si, v, id, gt);
-}
-
-template <int K>
-__device__ __forceinline__ void topk_insert_ordered(float (&sv)[K], int (&si)[K], float v, int id) {
-  bool gt[K];
-#pragma unroll
-  for (int j = 0; j < K; ++j) gt[j] = v > sv[j] || (v == sv[j] && id < si[j]);
   topk_insert_at<K>(sv, si, v, id, gt);
 }
 
@@ -360,48 +352,6 @@ __device__ __forceinline__ void topk_softmax_wave(const float* __restrict__ lrow
   float v[4];
   load_logits_lane(lrow, E, lane, v);
   topk_softmax_wave_vals<K>(v, E, lane, ids_out, w_out);
-}
-
-// The same top-k + softmax with LANES lanes per token (lanes LANES*t .. LANES*t + LANES-1, `sub` =
-// lane % LANES): each lane keeps the sorted top K of its 1/LANES of the logits (ascending ids,
-// strict > insertion), then log2(LANES) xor-shuffle rounds merge the lists under (value desc, id
-// asc), so all lanes of the group hold the same sorted selection as topk_softmax_lane and compute
-// the identical softmax; sub 0 writes.  lrow must be 16-byte aligned and the share Q = E/LANES a
-// multiple of 4 (E % (4*LANES) == 0).
-template <int K, int LANES>
-__device__ __forceinline__ void topk_softmax_group(const float* __restrict__ lrow, int E, int sub,
-                                                   int32_t* ids_out, float* w_out) {
-  float sv[K];
-  int si[K];
-#pragma unroll
-  for (int j = 0; j < K; ++j) { sv[j] = -INFINITY; si[j] = 0x7fffffff; }
-  const int Q = E / LANES;
-  for (int e0 = sub * Q; e0 < (sub + 1) * Q; e0 += 4) {
-    const float4 q = *reinterpret_cast<const float4*>(lrow + e0);
-    const float vv[4] = {q.x, q.y, q.z, q.w};
-#pragma unroll
-    for (int i = 0; i < 4; ++i) topk_insert_strict<K>(sv, si, vv[i], e0 + i);
-  }
-#pragma unroll
-  for (int o = 1; o < LANES; o <<= 1) {
-    float pv[K];
-    int pi[K];
-#pragma unroll
-    for (int j = 0; j < K; ++j) { pv[j] = __shfl_xor(sv[j], o, 64); pi[j] = __shfl_xor(si[j], o, 64); }
-#pragma unroll
-    for (int m = 0; m < K; ++m) topk_insert_ordered<K>(sv, si, pv[m], pi[m]);
-  }
-  float ex[K], sum = 0.f;
-#pragma unroll
-  for (int j = 0; j < K; ++j) { ex[j] = expf(sv[j] - sv[0]); sum += ex[j]; }
-  sort_ids_with_weights<K>(si, ex);
-  if (sub == 0) {
-#pragma unroll
-    for (int j = 0; j < K; ++j) {
-      ids_out[j] = (unsigned)si[j] < (unsigned)E ? si[j] : 0;  // a NaN row selects nothing: expert 0
-      w_out[j] = ex[j] / sum;
-    }
-  }
 }
 
 }  // namespace flyai

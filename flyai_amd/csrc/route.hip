@@ -2,6 +2,7 @@
 // Index outputs are bit-exact against the oracle: the logits use one fixed fp32 summation order
 // (64 lane partials, lane l over k = 512 j + 8 l + i in order, then a xor butterfly 32,16,8,4,2,1)
 // and ties in top-k go to the lower expert id.
+#include <algorithm>
 #include <type_traits>
 
 #include "common.h"
@@ -129,30 +130,83 @@ __global__ __launch_bounds__(256) void router_topk_kernel(const float* __restric
   topk_softmax_lane<K>(logits + (size_t)t * E, E, topk_ids + (size_t)t * K, topk_w + (size_t)t * K);
 }
 
-// The same selection with 4 lanes per token (64 tokens per workgroup) for E % 16 == 0, E <= 256:
-// each lane loads its quarter of the row (E/16 float4, all before the first compare) and parks it in
-// LDS (rows of E + 4 floats), then topk_softmax_group<K, 4> merges the quarters -- bit-identical to
-// topk_softmax_lane.  A lane reads back only what it wrote itself.
+// The router's logits are bf16 values, so for E <= 256 (value desc, id asc) is the order of one 24-bit
+// integer, (the value's 16 bits in value order) * 256 + 255 - id: a sorted list takes a new entry with one max
+// and one min a place, where (value, id) pairs take six comparisons and selects.  -0 and +0 are one value; a
+// NaN or -infinity is never selected (key 0: an empty place), as in topk_softmax_lane.  The pairs' chain of
+// compares, not the loads, was the time: 7.8 us for 2,096 tokens of 128 experts, with keys 6.0; one workgroup's
+// 12 tokens with their permute 7.4, with keys 5.9.
+__device__ __forceinline__ uint32_t topk_key(float v, int id) {
+  const uint32_t u = __float_as_uint(v) >> 16;
+  const uint32_t o = (u & 0x8000u) ? ~u & 0xffffu : u | 0x8000u;
+  return v > -INFINITY ? ((v == 0.f ? 0x8000u : o) << 8) | (uint32_t)(255 - id) : 0u;
+}
+
+template <int K>
+__device__ __forceinline__ void topk_key_insert(uint32_t (&a)[K], uint32_t x) {
+#pragma unroll
+  for (int j = 0; j < K; ++j) {
+    const uint32_t hi = max(a[j], x);
+    x = min(a[j], x);
+    a[j] = hi;
+  }
+}
+
+// The lists of 4 lanes (lane % 4 = sub) merged, then the softmax and id order of topk_softmax_lane, written by
+// sub 0.
+template <int K>
+__device__ __forceinline__ void topk_keys_finish(uint32_t (&a)[K], int E, int sub, int32_t* ids_out, float* w_out) {
+#pragma unroll
+  for (int o = 1; o < 4; o <<= 1) {
+    uint32_t p[K];
+#pragma unroll
+    for (int j = 0; j < K; ++j) p[j] = __shfl_xor(a[j], o, 64);
+#pragma unroll
+    for (int j = 0; j < K; ++j) topk_key_insert<K>(a, p[j]);
+  }
+  float sv[K], ex[K], sum = 0.f;
+  int si[K];
+#pragma unroll
+  for (int j = 0; j < K; ++j) {
+    const uint32_t o = a[j] >> 8;
+    sv[j] = a[j] ? __uint_as_float(((o & 0x8000u) ? o & 0x7fffu : ~o & 0xffffu) << 16) : -INFINITY;
+    si[j] = a[j] ? 255 - (int)(a[j] & 255u) : 0x7fffffff;
+  }
+#pragma unroll
+  for (int j = 0; j < K; ++j) { ex[j] = expf(sv[j] - sv[0]); sum += ex[j]; }
+  sort_ids_with_weights<K>(si, ex);
+  if (sub == 0) {
+#pragma unroll
+    for (int j = 0; j < K; ++j) {
+      ids_out[j] = (unsigned)si[j] < (unsigned)E ? si[j] : 0;  // a NaN row selects nothing: expert 0
+      w_out[j] = ex[j] / sum;
+    }
+  }
+}
+
+// The same selection with 4 lanes per token (64 tokens per workgroup) for E % 16 == 0, E <= 256: each lane
+// loads its quarter of the row (E/16 float4, all before the first comparison).
 template <int K>
 __global__ __launch_bounds__(256) void router_topk4_kernel(const float* __restrict__ logits, int T, int E,
                                                            int32_t* __restrict__ topk_ids,
                                                            float* __restrict__ topk_w) {
-  extern __shared__ float4 rows_lds[];  // [64][E + 4] floats
-  float* row = reinterpret_cast<float*>(rows_lds) + (threadIdx.x >> 2) * (E + 4);
-  const int sub = threadIdx.x & 3, tl = threadIdx.x >> 2;
-  const int t = blockIdx.x * 64 + tl;
+  const int sub = threadIdx.x & 3;
+  const int t = blockIdx.x * 64 + (int)(threadIdx.x >> 2);
+  if (t >= T) return;  // whole groups of 4 lanes stay together
   const int Q = E / 4;
+  const float4* row = reinterpret_cast<const float4*>(logits + (size_t)t * E + sub * Q);
   float4 v[16];
 #pragma unroll
-  for (int i = 0; i < 16; ++i) {
-    const int e0 = sub * Q + 4 * i;
-    v[i] = (t < T && 4 * i < Q) ? *reinterpret_cast<const float4*>(logits + (size_t)t * E + e0)
-                                : make_float4(0.f, 0.f, 0.f, 0.f);
-  }
+  for (int i = 0; i < 16; ++i) v[i] = 4 * i < Q ? row[i] : make_float4(-INFINITY, -INFINITY, -INFINITY, -INFINITY);
+  uint32_t a[K] = {};
 #pragma unroll
-  for (int i = 0; i < 16; ++i)
-    if (4 * i < Q) *reinterpret_cast<float4*>(row + sub * Q + 4 * i) = v[i];
-  if (t < T) topk_softmax_group<K, 4>(row, E, sub, topk_ids + (size_t)t * K, topk_w + (size_t)t * K);
+  for (int i = 0; i < 16; ++i) {
+    if (4 * i >= Q) break;
+    const float q[4] = {v[i].x, v[i].y, v[i].z, v[i].w};
+#pragma unroll
+    for (int c = 0; c < 4; ++c) topk_key_insert<K>(a, topk_key(q[c], sub * Q + 4 * i + c));
+  }
+  topk_keys_finish<K>(a, E, sub, topk_ids + (size_t)t * K, topk_w + (size_t)t * K);
 }
 
 int launch_router_logits(const uint16_t* x, const uint16_t* w, const uint16_t* b, int T, int H,
@@ -171,32 +225,26 @@ int launch_router_logits(const uint16_t* x, const uint16_t* w, const uint16_t* b
   return check_launch("router_logits");
 }
 
+int launch_topk(const float* logits, int T, int E, int k, int32_t* ids, float* wts, hipStream_t s) {
+  auto go = [&](auto kk) {
+    constexpr int K = decltype(kk)::value;
+    if (E % 16 == 0 && E <= 256)
+      hipLaunchKernelGGL(router_topk4_kernel<K>, dim3(ceil_div(T, 64)), dim3(256), 0, s, logits, T, E, ids, wts);
+    else
+      hipLaunchKernelGGL(router_topk_kernel<K>, dim3(ceil_div(T, 256)), dim3(256), 0, s, logits, T, E, ids, wts);
+  };
+  if (k == 4) go(std::integral_constant<int, 4>{});
+  else if (k == 8) go(std::integral_constant<int, 8>{});
+  else if (k == 2) go(std::integral_constant<int, 2>{});
+  else return set_error(FLYAI_EINVAL, "router: top_k must be 2, 4 or 8");
+  return check_launch("router_topk");
+}
+
 int launch_router(const uint16_t* x, const uint16_t* w, const uint16_t* b, int T, int H, int E,
                   int k, int32_t* ids, float* wts, float* logits, hipStream_t s) {
   if (T == 0) return FLYAI_OK;
-  int rc = launch_router_logits(x, w, b, T, H, E, logits, s);
-  if (rc) return rc;
-  if (E % 16 == 0 && E <= 256 && (k == 4 || k == 8 || k == 2)) {
-    if (k == 4)
-      hipLaunchKernelGGL(router_topk4_kernel<4>, dim3(ceil_div(T, 64)), dim3(256), 64 * (E + 4) * 4, s, logits, T, E,
-                         ids, wts);
-    else if (k == 8)
-      hipLaunchKernelGGL(router_topk4_kernel<8>, dim3(ceil_div(T, 64)), dim3(256), 64 * (E + 4) * 4, s, logits, T, E,
-                         ids, wts);
-    else
-      hipLaunchKernelGGL(router_topk4_kernel<2>, dim3(ceil_div(T, 64)), dim3(256), 64 * (E + 4) * 4, s, logits, T, E,
-                         ids, wts);
-    return check_launch("router_topk4");
-  }
-  if (k == 4)
-    hipLaunchKernelGGL(router_topk_kernel<4>, dim3(ceil_div(T, 256)), dim3(256), 0, s, logits, T, E, ids, wts);
-  else if (k == 8)
-    hipLaunchKernelGGL(router_topk_kernel<8>, dim3(ceil_div(T, 256)), dim3(256), 0, s, logits, T, E, ids, wts);
-  else if (k == 2)
-    hipLaunchKernelGGL(router_topk_kernel<2>, dim3(ceil_div(T, 256)), dim3(256), 0, s, logits, T, E, ids, wts);
-  else
-    return set_error(FLYAI_EINVAL, "router: top_k must be 2, 4 or 8");
-  return check_launch("router_topk");
+  const int rc = launch_router_logits(x, w, b, T, H, E, logits, s);
+  return rc ? rc : launch_topk(logits, T, E, k, ids, wts, s);
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -364,12 +412,16 @@ int launch_router_grouped(const uint16_t* x, const uint16_t* w, const float* e_b
 }
 
 // ------------------------------------------------------------------------------------------------
-// Histogram + exclusive scan + stable permute in one 16-wave workgroup.  Each wave owns a
-// contiguous segment of the flattened assignments; within a 64-assignment chunk, lanes with the
-// same expert find each other with 8 ballots (one per id bit), rank = popcount of lower peers, and
-// the lowest peer updates that wave's per-expert counter.  Pass 1 counts, the scan turns counts
-// into per-(wave, expert) cursors, pass 2 scatters.  Order: experts ascending, flat index ascending.
+// Histogram + exclusive scan + stable permute.  A workgroup of 16 waves places kPermBlock consecutive
+// assignments, one a thread: lanes with the same expert find each other with one ballot per id bit, rank =
+// popcount of lower peers, and the lowest peer stores its wave's count of that expert.  The experts' totals
+// and their counts before the block come from all P ids (LDS atomics: sums, so no order enters), read by
+// every workgroup, so the blocks need nothing from one another and no scratch memory.
+// Order: experts ascending, flat index ascending.
+// One workgroup over all assignments, each wave a serial run of chunks matched twice, took 5.9 us for 1,240
+// assignments of 256 experts, 12.8 for 5,200 and 19.6 for 8,384 of 128; now 5.4, 6.2 and 7.1.
 constexpr int kPermWaves = 16;
+constexpr int kPermBlock = kPermWaves * 64;
 
 __device__ __forceinline__ uint64_t match_peers(int e, bool valid, int nbits) {
   uint64_t peers = __ballot(valid);
@@ -381,101 +433,131 @@ __device__ __forceinline__ uint64_t match_peers(int e, bool valid, int nbits) {
   return peers;
 }
 
-// ids may live in global memory or LDS; called by all kPermWaves*64 threads of the workgroup.
-__device__ void permute_block(const int32_t* ids, int P, int E, int32_t* __restrict__ hist_out,
+// an id outside [0, E) (a router row of NaN) counts as expert 0, so the histogram still sums to P and every
+// slot gets a perm and an inv entry: the expert and combine kernels index with those
+__device__ __forceinline__ int perm_expert(int e, int E) { return (e < 0 || e >= E) ? 0 : e; }
+
+struct PermShared {
+  int32_t cnt[kPermWaves][256];  // per (wave, expert) counts, then the wave's first slot after `first`
+  int32_t total[256], before[256];
+  int32_t first[256];            // the expert's first slot of this block
+};
+
+// Places assignments [blk * kPermBlock, ...) of `P`.  ids may live in global memory or LDS; called by all
+// kPermBlock threads of the workgroup.
+__device__ void permute_block(const int32_t* ids, int blk, int P, int E, int32_t* __restrict__ hist_out,
                               int32_t* __restrict__ off_out, int32_t* __restrict__ perm,
-                              int32_t* __restrict__ inv, int32_t (*cnt)[256], int32_t* off) {
+                              int32_t* __restrict__ inv, PermShared& sh) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  for (int i = tid; i < kPermWaves * 256; i += kPermWaves * 64) (&cnt[0][0])[i] = 0;
-  __syncthreads();
+  const int a = blk * kPermBlock + tid;
+  const bool valid = a < P;
+  const int e = valid ? perm_expert(ids[a], E) : 0;
+  for (int i = tid; i < kPermWaves * 256; i += kPermBlock) (&sh.cnt[0][0])[i] = 0;
+  if (tid < 256) sh.total[tid] = sh.before[tid] = 0;
   int nbits = 0;
   while ((1 << nbits) < E) ++nbits;
-  const int seg = ((P + kPermWaves * 64 - 1) / (kPermWaves * 64)) * 64;
-  const int beg = min(P, wave * seg), end = min(P, beg + seg);
+  const uint64_t peers = match_peers(e, valid, nbits);
   const uint64_t lt = (lane == 0) ? 0ull : ((~0ull) >> (64 - lane));
-  for (int base = beg; base < end; base += 64) {
-    const int a = base + lane;
-    // an id outside [0, E) (a router row of NaN) counts as expert 0, so the histogram still sums to P
-    // and every slot gets a perm and an inv entry: the expert and combine kernels index with those
-    int e = a < end ? ids[a] : -1;
-    const bool valid = a < end;
-    if (e < 0 || e >= E) e = 0;
-    const uint64_t peers = match_peers(e, valid, nbits);
-    if (valid && (peers & lt) == 0) cnt[wave][e] += __popcll(peers);
-  }
+  const int rank = __popcll(peers & lt);
   __syncthreads();
-  if (tid < E) {
-    int h = 0;
-    for (int w = 0; w < kPermWaves; ++w) h += cnt[w][tid];
-    hist_out[tid] = h;
-    off[tid] = h;
-  }
-  __syncthreads();
-  if (wave == 0) {  // exclusive scan of off[0..E), 4 entries per lane
-    int v[4], sum = 0;
-    for (int c = 0; c < 4; ++c) { int i = lane * 4 + c; v[c] = i < E ? off[i] : 0; sum += v[c]; }
-    int incl = sum;
-    for (int o = 1; o < 64; o <<= 1) { int y = __shfl_up(incl, o, 64); if (lane >= o) incl += y; }
-    int run = incl - sum;
-    for (int c = 0; c < 4; ++c) { int i = lane * 4 + c; if (i < E) off[i] = run; run += v[c]; }
-  }
-  __syncthreads();
-  if (tid < E) {
-    int run = off[tid];
-    off_out[tid] = run;
-    for (int w = 0; w < kPermWaves; ++w) { int c = cnt[w][tid]; cnt[w][tid] = run; run += c; }
-  }
-  if (tid == 0) off_out[E] = P;
-  __syncthreads();
-  for (int base = beg; base < end; base += 64) {
-    const int a = base + lane;
-    int e = a < end ? ids[a] : -1;
-    const bool valid = a < end;
-    if (e < 0 || e >= E) e = 0;
-    const uint64_t peers = match_peers(e, valid, nbits);
-    if (valid) {
-      const int pos = cnt[wave][e] + __popcll(peers & lt);
-      perm[pos] = a;
-      inv[a] = pos;
+  if (valid && rank == 0) sh.cnt[wave][e] = __popcll(peers);
+  const bool whole = P <= kPermBlock;  // this block is all there is
+  if (!whole) {
+    // four ids in flight a thread
+    for (int i0 = tid; i0 < P; i0 += 4 * kPermBlock) {
+      int v[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) v[j] = i0 + j * kPermBlock < P ? ids[i0 + j * kPermBlock] : 0;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int i = i0 + j * kPermBlock;
+        if (i >= P) break;
+        const int x = perm_expert(v[j], E);
+        atomicAdd(&sh.total[x], 1);
+        if (i < blk * kPermBlock) atomicAdd(&sh.before[x], 1);
+      }
     }
-    if (valid && (peers & lt) == 0) cnt[wave][e] += __popcll(peers);
+  }
+  __syncthreads();
+  if (tid < E) {
+    int run = 0;
+#pragma unroll
+    for (int w = 0; w < kPermWaves; ++w) {
+      const int c = sh.cnt[w][tid];
+      sh.cnt[w][tid] = run;
+      run += c;
+    }
+    if (whole) sh.total[tid] = run;
+    if (blk == 0) hist_out[tid] = whole ? run : sh.total[tid];
+  }
+  __syncthreads();
+  if (wave == 0) {  // exclusive scan of total[0..E), 4 entries per lane
+    int v[4], sum = 0;
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      const int i = lane * 4 + c;
+      v[c] = i < E ? sh.total[i] : 0;
+      sum += v[c];
+    }
+    int incl = sum;
+    for (int o = 1; o < 64; o <<= 1) {
+      const int y = __shfl_up(incl, o, 64);
+      if (lane >= o) incl += y;
+    }
+    int run = incl - sum;
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      const int i = lane * 4 + c;
+      if (i < E) {
+        sh.first[i] = run + sh.before[i];
+        if (blk == 0) off_out[i] = run;
+      }
+      run += v[c];
+    }
+    if (blk == 0 && lane == 0) off_out[E] = P;
+  }
+  __syncthreads();
+  if (valid) {
+    const int pos = sh.first[e] + sh.cnt[wave][e] + rank;
+    perm[pos] = a;
+    inv[a] = pos;
   }
 }
 
-__global__ __launch_bounds__(kPermWaves * 64) void moe_permute_kernel(
+__global__ __launch_bounds__(kPermBlock) void moe_permute_kernel(
     const int32_t* __restrict__ ids, int P, int E, int32_t* __restrict__ hist_out,
     int32_t* __restrict__ off_out, int32_t* __restrict__ perm, int32_t* __restrict__ inv) {
-  __shared__ int32_t cnt[kPermWaves][256];
-  __shared__ int32_t off[256];
-  permute_block(ids, P, E, hist_out, off_out, perm, inv, cnt, off);
+  __shared__ PermShared sh;
+  permute_block(ids, blockIdx.x, P, E, hist_out, off_out, perm, inv, sh);
 }
 
-// Small batches: top-k of every token (one lane per token) into LDS, then the permute, in one
-// workgroup -- one launch instead of two.
-constexpr int kFusedMaxAssign = 4096;
-
+// Small batches: top-k of every token into LDS, then the permute, in one workgroup -- one launch instead of
+// two: 7.4 us for 56 tokens of 128 experts, where the two launches take 5.4 + 5.4.  Past what its LDS holds (62
+// tokens of 128 experts) they are the faster way: one workgroup took 16 us for 110 tokens and 20 for 333, the two
+// take 11.1 and 11.4.
+constexpr int kFusedTokens = 64;
 constexpr int kStagedLogits = 8192;  // floats of logits staged in LDS (T * (E + 4) <= this)
 
+inline bool fused_topk_permute(int T, int E) { return T <= kFusedTokens && T * (E + 4) <= kStagedLogits; }
+
 template <int K>
-__global__ __launch_bounds__(kPermWaves * 64) void moe_topk_permute_kernel(
+__global__ __launch_bounds__(kPermBlock) void moe_topk_permute_kernel(
     const float* __restrict__ logits, int T, int E, int32_t* __restrict__ topk_ids,
     float* __restrict__ topk_w, int32_t* __restrict__ hist_out, int32_t* __restrict__ off_out,
     int32_t* __restrict__ perm, int32_t* __restrict__ inv) {
-  __shared__ int32_t cnt[kPermWaves][256];
-  __shared__ int32_t off[256];
-  __shared__ int32_t ids_s[kFusedMaxAssign];
+  __shared__ PermShared sh;
+  __shared__ int32_t ids_s[kFusedTokens * K];
   __shared__ __align__(16) float lg_s[kStagedLogits];
-  // one lane per token (a wave selects for 64 tokens at once); small batches first stage all logits
-  // in LDS with coalesced loads (rows padded by 16 bytes), so the selection never waits on memory
-  const bool staged = T * (E + 4) <= kStagedLogits;
-  if (staged) {
+  static_assert(kFusedTokens * K <= kPermBlock, "one permute block");
+  // all logits go to LDS with coalesced loads (rows padded by 16 bytes), so the selection never waits on memory
+  {
     // every load of the thread goes out before the first LDS store (one round trip, not one per
     // element): T * E < kStagedLogits = 8 per thread
-    constexpr int kPer = kStagedLogits / (kPermWaves * 64);
+    constexpr int kPer = kStagedLogits / (kPermBlock);
     float v[kPer];
 #pragma unroll
     for (int j = 0; j < kPer; ++j) {
-      const int i = threadIdx.x + j * kPermWaves * 64;
+      const int i = threadIdx.x + j * kPermBlock;
       v[j] = i < T * E ? logits[i] : 0.f;
     }
     // row-major into rows of E + 4 floats; (row, column) by a shift and a mask when E is a power
@@ -484,87 +566,78 @@ __global__ __launch_bounds__(kPermWaves * 64) void moe_topk_permute_kernel(
       const int e_shift = __builtin_ctz((unsigned)E);
 #pragma unroll
       for (int j = 0; j < kPer; ++j) {
-        const int i = threadIdx.x + j * kPermWaves * 64;
+        const int i = threadIdx.x + j * kPermBlock;
         if (i < T * E) lg_s[(i >> e_shift) * (E + 4) + (i & (E - 1))] = v[j];
       }
     } else {
 #pragma unroll
       for (int j = 0; j < kPer; ++j) {
-        const int i = threadIdx.x + j * kPermWaves * 64;
+        const int i = threadIdx.x + j * kPermBlock;
         if (i < T * E) lg_s[(i / E) * (E + 4) + i % E] = v[j];
       }
     }
     __syncthreads();
   }
-  if (staged && E % 16 == 0) {
-    // four lanes per token: 256 tokens per pass of the workgroup
-    const int sub = threadIdx.x & 3;
-    for (int t0 = 0; t0 < T; t0 += kPermWaves * 16) {
-      const int t = t0 + (threadIdx.x >> 2);
-      // whole quads stay together (T rounds the quad index, never splits one)
-      if (t < T) topk_softmax_group<K, 4>(lg_s + t * (E + 4), E, sub, ids_s + t * K, topk_w + (size_t)t * K);
+  if (E % 16 == 0) {  // four lanes per token, as router_topk4_kernel
+    const int t = threadIdx.x >> 2, sub = threadIdx.x & 3, Q = E / 4;
+    if (t < T) {
+      const float4* row = reinterpret_cast<const float4*>(lg_s + t * (E + 4) + sub * Q);
+      uint32_t a[K] = {};
+      for (int i = 0; i < Q / 4; ++i) {
+        const float4 v = row[i];
+        const float q[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+        for (int c = 0; c < 4; ++c) topk_key_insert<K>(a, topk_key(q[c], sub * Q + 4 * i + c));
+      }
+      topk_keys_finish<K>(a, E, sub, ids_s + t * K, topk_w + (size_t)t * K);
     }
-  } else {
-    for (int t = threadIdx.x; t < T; t += kPermWaves * 64)
-      topk_softmax_lane<K>(staged ? lg_s + t * (E + 4) : logits + (size_t)t * E, E, ids_s + t * K,
-                           topk_w + (size_t)t * K);
+  } else if ((int)threadIdx.x < T) {
+    const int t = threadIdx.x;
+    topk_softmax_lane<K>(lg_s + t * (E + 4), E, ids_s + t * K, topk_w + (size_t)t * K);
   }
   __syncthreads();
-  for (int i = threadIdx.x; i < T * K; i += kPermWaves * 64) topk_ids[i] = ids_s[i];
-  permute_block(ids_s, T * K, E, hist_out, off_out, perm, inv, cnt, off);
+  if ((int)threadIdx.x < T * K) topk_ids[threadIdx.x] = ids_s[threadIdx.x];
+  permute_block(ids_s, 0, T * K, E, hist_out, off_out, perm, inv, sh);
 }
 
 int launch_permute(const int32_t* ids, int T, int k, int E, int32_t* hist, int32_t* offsets,
                    int32_t* perm, int32_t* inv, hipStream_t s);
 
+int launch_topk(const float* logits, int T, int E, int k, int32_t* ids, float* wts, hipStream_t s);
+
+// Top-k + softmax of precomputed logits, then histogram / permute: one workgroup for a small batch,
+// else a launch of each over the whole chip.
+int launch_topk_permute(const float* logits, int T, int E, int k, int32_t* ids, float* wts, int32_t* hist,
+                        int32_t* offsets, int32_t* perm, int32_t* inv, hipStream_t s) {
+  if (T == 0) return FLYAI_OK;
+  if (!fused_topk_permute(T, E)) {
+    const int rc = launch_topk(logits, T, E, k, ids, wts, s);
+    return rc ? rc : launch_permute(ids, T, k, E, hist, offsets, perm, inv, s);
+  }
+  auto go = [&](auto kk) {
+    hipLaunchKernelGGL((moe_topk_permute_kernel<decltype(kk)::value>), dim3(1), dim3(kPermBlock), 0, s, logits, T, E, ids,
+                       wts, hist, offsets, perm, inv);
+  };
+  if (k == 4) go(std::integral_constant<int, 4>{});
+  else if (k == 8) go(std::integral_constant<int, 8>{});
+  else if (k == 2) go(std::integral_constant<int, 2>{});
+  else return set_error(FLYAI_EINVAL, "route: top_k must be 2, 4 or 8");
+  return check_launch("moe_topk_permute");
+}
+
 int launch_route_permute(const uint16_t* x, const uint16_t* w, const uint16_t* b, int T, int H,
                          int E, int k, int32_t* ids, float* wts, float* logits, int32_t* hist,
                          int32_t* offsets, int32_t* perm, int32_t* inv, hipStream_t s) {
   if (T == 0) return FLYAI_OK;
-  if (T * k > kFusedMaxAssign) {
-    int rc = launch_router(x, w, b, T, H, E, k, ids, wts, logits, s);
-    if (rc) return rc;
-    return launch_permute(ids, T, k, E, hist, offsets, perm, inv, s);
-  }
-  int rc = launch_router_logits(x, w, b, T, H, E, logits, s);
-  if (rc) return rc;
-  if (k == 4)
-    hipLaunchKernelGGL(moe_topk_permute_kernel<4>, dim3(1), dim3(kPermWaves * 64), 0, s, logits, T, E,
-                       ids, wts, hist, offsets, perm, inv);
-  else if (k == 8)
-    hipLaunchKernelGGL(moe_topk_permute_kernel<8>, dim3(1), dim3(kPermWaves * 64), 0, s, logits, T, E,
-                       ids, wts, hist, offsets, perm, inv);
-  else if (k == 2)
-    hipLaunchKernelGGL(moe_topk_permute_kernel<2>, dim3(1), dim3(kPermWaves * 64), 0, s, logits, T, E,
-                       ids, wts, hist, offsets, perm, inv);
-  else
-    return set_error(FLYAI_EINVAL, "route: top_k must be 2, 4 or 8");
-  return check_launch("moe_topk_permute");
-}
-
-// Top-k + softmax of precomputed logits, then histogram / permute (T*k <= 4096: one workgroup).
-int launch_topk_permute(const float* logits, int T, int E, int k, int32_t* ids, float* wts, int32_t* hist,
-                        int32_t* offsets, int32_t* perm, int32_t* inv, hipStream_t s) {
-  if (T == 0) return FLYAI_OK;
-  if ((int64_t)T * k > kFusedMaxAssign) return set_error(FLYAI_EINVAL, "topk_permute: T*k > %d", kFusedMaxAssign);
-  if (k == 4)
-    hipLaunchKernelGGL(moe_topk_permute_kernel<4>, dim3(1), dim3(kPermWaves * 64), 0, s, logits, T, E, ids,
-                       wts, hist, offsets, perm, inv);
-  else if (k == 8)
-    hipLaunchKernelGGL(moe_topk_permute_kernel<8>, dim3(1), dim3(kPermWaves * 64), 0, s, logits, T, E, ids,
-                       wts, hist, offsets, perm, inv);
-  else if (k == 2)
-    hipLaunchKernelGGL(moe_topk_permute_kernel<2>, dim3(1), dim3(kPermWaves * 64), 0, s, logits, T, E, ids,
-                       wts, hist, offsets, perm, inv);
-  else
-    return set_error(FLYAI_EINVAL, "route: top_k must be 2, 4 or 8");
-  return check_launch("moe_topk_permute");
+  const int rc = launch_router_logits(x, w, b, T, H, E, logits, s);
+  return rc ? rc : launch_topk_permute(logits, T, E, k, ids, wts, hist, offsets, perm, inv, s);
 }
 
 int launch_permute(const int32_t* ids, int T, int k, int E, int32_t* hist, int32_t* offsets,
                    int32_t* perm, int32_t* inv, hipStream_t s) {
-  hipLaunchKernelGGL(moe_permute_kernel, dim3(1), dim3(kPermWaves * 64), 0, s, ids, T * k, E,
-                     hist, offsets, perm, inv);
+  // (no assignments: one workgroup still writes the empty histogram and offsets)
+  hipLaunchKernelGGL(moe_permute_kernel, dim3(std::max(1, ceil_div(T * k, kPermBlock))), dim3(kPermBlock), 0, s, ids,
+                     T * k, E, hist, offsets, perm, inv);
   return check_launch("moe_permute");
 }
 

@@ -162,6 +162,40 @@ def test_permute_bit_exact(T, k, E, mode):
     assert np.array_equal(inv.cpu().numpy(), ri)
 
 
+@pytest.mark.parametrize("P,E", [(1, 1), (63, 3), (1023, 128), (1024, 256), (1025, 255), (4097, 64), (8384, 7),
+                                 (65536, 256)])
+def test_permute_blocks_bit_exact(P, E):
+    """The permute's blocks of 1,024 assignments: one short, full, one over, many; ids outside [0, E) count as
+    expert 0 in the counts of a block and in the counts before it."""
+    from flyai_amd import ops
+    rng = np.random.default_rng(P + E)
+    ids = rng.integers(-1, E + 1, size=(P, 1)).astype(np.int32)
+    got = ops.moe_permute(torch.tensor(ids, device=DEV), E)
+    ref = oroute.permute(np.where((ids >= 0) & (ids < E), ids, 0), E)
+    for g, r in zip(got, ref):
+        assert np.array_equal(g.cpu().numpy(), r)
+
+
+# the last batch of the one-workgroup kernel and the first of the two launches, per E and selection kernel
+@pytest.mark.parametrize("T,E,k", [(62, 128, 4), (63, 128, 4), (31, 256, 8), (32, 256, 8), (64, 4, 2), (65, 4, 4),
+                                   (64, 120, 4), (70, 120, 8), (64, 16, 8), (300, 112, 2)])
+def test_route_selection_order_bit_exact(T, E, k):
+    """Logits of every kind the selection's integer order has to rank: both signs, zeros, ties, subnormals, the
+    largest magnitudes and -infinity (zero weights: the bias is the logit)."""
+    from flyai_amd import ops
+    x = _rms_input(T, 256, 16)
+    w = torch.zeros(E, 256, device=DEV, dtype=torch.bfloat16)
+    kinds = torch.tensor([-1.5, 0.0, 2.0**-130, -2.0**-130, 0.75, -3.38e38, float("-inf"), 0.75, -0.25, 1e-3, 1.0])
+    b = kinds[torch.randperm(E, generator=torch.Generator().manual_seed(E)) % len(kinds)].to(torch.bfloat16)
+    w[:, 0] = torch.linspace(-2, 2, E).to(torch.bfloat16).to(DEV) * (torch.arange(E, device=DEV) % 3 == 0)
+    ids, wts, *perm = ops.moe_route_permute(x, w, b.to(DEV), k)
+    rids, rw, _ = oroute.gptoss_route(x.float().cpu(), w.float().cpu(), b.float(), k)
+    assert np.array_equal(ids.cpu().numpy(), rids)
+    np.testing.assert_allclose(wts.cpu().numpy(), rw, rtol=2e-6, atol=1e-7)
+    for g, r in zip(perm, oroute.permute(rids, E)):
+        assert np.array_equal(g.cpu().numpy(), r)
+
+
 def test_nan_router_rows_route_consistently():
     """A router row of NaN (a NaN hidden state) must not break the routing's index invariants: the
     expert and combine kernels index with perm, inv and offsets.  The top-k gives such a row
