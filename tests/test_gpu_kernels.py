@@ -704,6 +704,36 @@ def test_dense_and_row_pass_experts_bit_identical():
             assert torch.equal(y_a[ra], y_b[rb]), f"expert {e}, tokens {sel}: down differs"
 
 
+@pytest.mark.parametrize("E,groups", [(130, {0: 2, 63: 1, 64: 9, 127: 1, 128: 3, 129: 1}), (130, {129: 1}), (4, {2: 5}),
+                                      (64, {63: 17}), (200, {e: 1 for e in range(3, 200, 2)})])
+def test_few_groups_experts_bit_identical(E, groups):
+    """The row-pass kernel's workgroups are counted over the groups that have rows (128 experts counted at a
+    time): each group's h and y equal that expert's alone in a one-expert call, bit for bit."""
+    from flyai_amd import ops
+    from flyai_amd.weights import GptOssShape, synthetic_moe
+    H, I = 160, 96
+    m = synthetic_moe(GptOssShape(hidden=H, intermediate=I, n_experts=E), _gen(63), DEV)
+    w13 = ops.mxfp4_repack(m["w13_blocks"], m["w13_scales"])
+    w2 = ops.mxfp4_repack(m["w2_blocks"], m["w2_scales"])
+    ids = torch.tensor([e for e, n in groups.items() for _ in range(n)], dtype=torch.int32, device=DEV)[:, None]
+    x = _rms_input(len(ids), H, 64)
+    _, off, perm, _ = ops.moe_permute(ids, E)
+    h = ops.moe_gate_up(x, perm, off, 1, w13, m["b13"], E, I)
+    y = ops.moe_down(h, off, w2, m["b2"], E, H)
+    lo = 0
+    for e, n in groups.items():
+        one = [ops.mxfp4_repack(m[f"{w}_blocks"][e:e + 1].contiguous(), m[f"{w}_scales"][e:e + 1].contiguous())
+               for w in ("w13", "w2")]
+        for r in range(lo, lo + n, 5):  # at most 5 rows: the row-pass kernel
+            rows = x[r:min(r + 5, lo + n)].contiguous()
+            _, off1, perm1, _ = ops.moe_permute(torch.zeros(len(rows), 1, dtype=torch.int32, device=DEV), 1)
+            h1 = ops.moe_gate_up(rows, perm1, off1, 1, one[0], m["b13"][e:e + 1].contiguous(), 1, I)
+            y1 = ops.moe_down(h1, off1, one[1], m["b2"][e:e + 1].contiguous(), 1, H)
+            assert torch.equal(h1.view(torch.int16), h[r:r + len(rows)].view(torch.int16)), f"gate_up of expert {e}"
+            assert torch.equal(y1.view(torch.int32), y[r:r + len(rows)].view(torch.int32)), f"down of expert {e}"
+        lo += n
+
+
 @pytest.mark.parametrize("H,I", [(2880, 2880), (128, 160), (544, 2048)])
 def test_medium_group_experts_bit_identical(H, I):
     """A batch of 6 to 18 rows per expert on average runs the medium-group kernel; the same rows in batches
