@@ -22,151 +22,119 @@ int launch_rmsnorm(const uint16_t* x, const float* w, int T, int H, float eps, u
 }
 
 // ---- bf16 projections: split-K partial GEMM + fused finalize kernels -------------------------------
-// gemm_splitk: workgroup = 4 waves on 4 consecutive 16-feature tiles and one K slice of kKQW groups
+// gemm_splitk: workgroup = 4 or 8 waves on as many consecutive 16-feature tiles and one K slice of kKQW groups
 // of 128.  MFMA step j of group q takes, in lane (r, g), K = 128q + 32j + 8g .. +7 for both operands
 // (any K order shared by the two operands is valid), so each weight load instruction reads one
 // whole 64-byte run of each of its 16 rows.  The activation slice (64 rows x 512 K, bf16) is staged once in LDS; each wave issues all
 // of its weight loads for the slice before its first MFMA (a single HBM round trip per wave) and
 // writes fp32 partial sums part[slice][row][feature].  A finalize kernel adds the slices in slice
 // order (so the result is independent of timing), the bias, and the fused epilogue.
+typedef float f32x4_dw __attribute__((ext_vector_type(4), aligned(4)));  // partials are 4-byte aligned,
+typedef uint16_t u16x4_h __attribute__((ext_vector_type(4), aligned(2)));  // bf16 tensors 2-byte
 constexpr int kKQW = 4;       // K groups of 128 per slice
 constexpr int kGemmRows = 64; // activation rows per pass
 
-__global__ __launch_bounds__(256) void gemm_splitk_bf16_kernel(
+// More rows than a pass: the weights stay in registers over the passes of 64 rows, and the next pass's activations
+// are loaded into registers under the current pass's MFMAs (one barrier pair a pass, on LDS only: the loads stay in
+// flight).  A pass used to be staged behind a barrier that drained every load, by workgroups of 64 features: the
+// two projections of 5,120 x 2,880 and 2,880 x 4,096 took 19.2 and 18.5 us at 137 rows, now 16.3 and 15.6; 24.9 and
+// 24.3 at 255, now 22.5 and 22.2.  Eight waves and 128 features read the activations half as often from L2; wider
+// waves (two feature tiles each) made no difference.  What is left past the weights' 5 us is the partial planes'
+// way out, about 4 us per 64 rows, which the slice order of the sums needs.
+// No load sits under a lane's branch: rows past M and features past N read a clamped one (their sums are not
+// stored), K past the row's end is replaced by zero in both operands.  With the loads predicated the weights' waited
+// for the activations' to return: 7.7 us for 1 row of either projection, 8.1 for 16; now 7.2 and 7.5.
+template <int WAVES>
+__global__ __launch_bounds__(64 * WAVES) void gemm_splitk_bf16_kernel(
     const uint16_t* __restrict__ x, const uint16_t* __restrict__ W, int M, int N, int K,
     float* __restrict__ part) {
-  __shared__ uint4 as[kGemmRows][kKQW * 16 + 1];  // 64 rows x 512 bf16, +16 B per row vs bank conflicts
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+  __shared__ u32x4 as[kGemmRows][kKQW * 16 + 1];  // 64 rows x 512 bf16, +16 B per row vs bank conflicts
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int r = lane & 15, g = lane >> 4;
-  const int nt = blockIdx.x * 4 + wave;
+  const int nt = blockIdx.x * WAVES + wave;
   const int slice = blockIdx.y;
   const int KQ = (K + 127) / 128;
   const int kq0 = slice * kKQW;
   const int nkq = min(kKQW, KQ - kq0);
-  const bool nval = nt * 16 < N;
   const int feat = nt * 16 + r;
-  typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
-  if (M <= kGemmRows) {
-    // One pass (decode-sized M): the activation slice's loads go out first, then the weights, so the
-    // LDS stores wait only for the activations (loads complete in issue order) and the L2 round trip
-    // for them overlaps the HBM fetch of the weights; the barrier then waits on LDS only.
-    constexpr int kPer = kGemmRows * kKQW * 16 / 256;  // 16-byte vectors per thread
-    u32x4 av[kPer];
+  // a wave loads whole rows of the slice (64 lanes x 16 bytes): row WAVES j + wave of the pass in load j
+  constexpr int kPer = kGemmRows / WAVES, kPerTile = 16 / WAVES;
+  static_assert(kKQW * 16 == 64, "one row of a slice is one wave load");
+  const int k = 128 * kq0 + 8 * lane;
+  const bool kval = k < K;
+  const uint16_t* xk = x + min(k, K - 8);
+  u32x4 av[kPer];
+  auto load_rows = [&](int m0) __attribute__((always_inline)) {
 #pragma unroll
-    for (int j = 0; j < kPer; ++j) {
-      const int i = j * 256 + (int)threadIdx.x;
-      const int row = i / (kKQW * 16), v = i % (kKQW * 16);
-      const int k = 128 * kq0 + 8 * v;
-      const bool ok = row < M && k < K;
-      av[j] = ok ? *reinterpret_cast<const u32x4*>(x + (size_t)row * K + k) : u32x4{0u, 0u, 0u, 0u};
-    }
-    asm volatile("" ::: "memory");  // keep the activation loads ahead of the weight loads
-    uint4 wv[kKQW][4];
+    for (int t = 0; t < kGemmRows / 16; ++t)
+      if (m0 + 16 * t < M) {
 #pragma unroll
-    for (int q = 0; q < kKQW; ++q) {
-      const int kb = 128 * (kq0 + q);
-      const bool ok = nval && q < nkq;
+        for (int j = t * kPerTile; j < (t + 1) * kPerTile; ++j)
+          av[j] = *reinterpret_cast<const u32x4*>(xk + (size_t)min(m0 + WAVES * j + wave, M - 1) * K);
+      }
+  };
+  auto store_rows = [&](int m0) __attribute__((always_inline)) {
+#pragma unroll
+    for (int t = 0; t < kGemmRows / 16; ++t)
+      if (m0 + 16 * t < M) {
+#pragma unroll
+        for (int j = t * kPerTile; j < (t + 1) * kPerTile; ++j)
+          as[WAVES * j + wave][lane] = kval ? av[j] : u32x4{0u, 0u, 0u, 0u};
+      }
+  };
+  // The activation slice's loads go out first, then the weights, so the LDS stores wait only for the activations
+  // (loads complete in issue order) and the L2 round trip for them overlaps the HBM fetch of the weights.
+  load_rows(0);
+  const uint16_t* wrow = W + (size_t)min(feat, N - 1) * K + 8 * g;
+  u32x4 wv[kKQW][4];
+#pragma unroll
+  for (int q = 0; q < kKQW; ++q)
+    if (q < nkq) {
 #pragma unroll
       for (int j = 0; j < 4; ++j)  // step j reads K kb + 32j .. +31 (K % 32 == 0)
-        wv[q][j] = ok && kb + 32 * j < K ? reinterpret_cast<const uint4*>(W + (size_t)feat * K + kb)[4 * j + g]
-                                         : make_uint4(0, 0, 0, 0);
+        wv[q][j] = *reinterpret_cast<const u32x4*>(wrow + min(128 * (kq0 + q) + 32 * j, K - 32));
     }
-#pragma unroll
-    for (int j = 0; j < kPer; ++j) {
-      const int i = j * 256 + (int)threadIdx.x;
-      *reinterpret_cast<u32x4*>(&as[i / (kKQW * 16)][i % (kKQW * 16)]) = av[j];
-    }
-    lds_barrier();
-    if (!nval) return;
-    const int mt_count = (M + 15) / 16;
-    f32x4_t acc[4] = {f32x4_t{0.f, 0.f, 0.f, 0.f}, f32x4_t{0.f, 0.f, 0.f, 0.f},
-                      f32x4_t{0.f, 0.f, 0.f, 0.f}, f32x4_t{0.f, 0.f, 0.f, 0.f}};
-#pragma unroll
-    for (int q = 0; q < kKQW; ++q) {
-      if (q >= nkq) break;
-#pragma unroll
-      for (int m = 0; m < 4; ++m) {
-        if (m >= mt_count) break;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const uint4 av4 = as[16 * m + r][q * 16 + 4 * j + g];
-          acc[m] = mfma16x16x32(as_bf16x8(av4), as_bf16x8(wv[q][j]), acc[m]);
-        }
-      }
-    }
-    float* pp = part + (size_t)slice * M * N;
-#pragma unroll
-    for (int m = 0; m < 4; ++m) {
-      if (m >= mt_count) break;
-#pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        const int row = 16 * m + 4 * g + v;
-        if (row < M) pp[(size_t)row * N + feat] = acc[m][v];
-      }
-    }
-    return;
-  }
-  // weights for the whole slice, issued up front (reused by every pass of 64 rows)
-  uint4 wv[kKQW][4];
-#pragma unroll
-  for (int q = 0; q < kKQW; ++q) {
-    const int kb = 128 * (kq0 + q);
-    const bool ok = nval && q < nkq;
-#pragma unroll
-    for (int j = 0; j < 4; ++j)  // step j reads K kb + 32j .. +31 (K % 32 == 0)
-      wv[q][j] = ok && kb + 32 * j < K ? reinterpret_cast<const uint4*>(W + (size_t)feat * K + kb)[4 * j + g]
-                                       : make_uint4(0, 0, 0, 0);
-  }
+  float* pp = part + (size_t)slice * M * N;
   for (int m0 = 0; m0 < M; m0 += kGemmRows) {
-    const int rows = min(kGemmRows, M - m0);
-    __syncthreads();
-    // the slice of A goes to LDS with loads batched 8 per thread (one round trip per batch);
-    // rows past the pass and K past the row end are stored as zero
-    for (int b0 = 0; b0 < kGemmRows * kKQW * 16; b0 += 8 * 256) {
-      u32x4 v8[8];
+    if (m0) lds_barrier();  // every wave has read the previous pass's rows
+    store_rows(m0);
+    if (m0 + kGemmRows < M) load_rows(m0 + kGemmRows);
+    lds_barrier();
+    // the row tiles of the pass as a constant: without branches between them their MFMA chains interleave
+    const auto pass = [&](auto tiles) __attribute__((always_inline)) {
+      constexpr int MT = decltype(tiles)::value;
+      f32x4_t acc[MT];
 #pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const int i = b0 + j * 256 + (int)threadIdx.x;
-        const int row = i / (kKQW * 16), v = i % (kKQW * 16);
-        const int k = 128 * kq0 + 8 * v;
-        const bool ok = row < rows && k < K;
-        const u32x4 val = *reinterpret_cast<const u32x4*>(x + (ok ? (size_t)(m0 + row) * K + k : 0));
-        v8[j] = ok ? val : u32x4{0u, 0u, 0u, 0u};
-      }
+      for (int m = 0; m < MT; ++m) acc[m] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const int i = b0 + j * 256 + (int)threadIdx.x;
-        *reinterpret_cast<u32x4*>(&as[i / (kKQW * 16)][i % (kKQW * 16)]) = v8[j];
-      }
-    }
-    __syncthreads();
-    if (!nval) continue;
-    const int mt_count = (rows + 15) / 16;
-    f32x4_t acc[4] = {f32x4_t{0.f, 0.f, 0.f, 0.f}, f32x4_t{0.f, 0.f, 0.f, 0.f},
-                      f32x4_t{0.f, 0.f, 0.f, 0.f}, f32x4_t{0.f, 0.f, 0.f, 0.f}};
-#pragma unroll
-    for (int q = 0; q < kKQW; ++q) {
-      if (q >= nkq) break;
-#pragma unroll
-      for (int m = 0; m < 4; ++m) {
-        if (m >= mt_count) break;
+      for (int q = 0; q < kKQW; ++q) {
+        if (q >= nkq) break;
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-          const uint4 av = as[16 * m + r][q * 16 + 4 * j + g];
-          acc[m] = mfma16x16x32(as_bf16x8(av), as_bf16x8(wv[q][j]), acc[m]);
+          const u32x4 w = 128 * (kq0 + q) + 32 * j < K ? wv[q][j] : u32x4{0u, 0u, 0u, 0u};
+#pragma unroll
+          for (int m = 0; m < MT; ++m)
+            acc[m] = mfma16x16x32(__builtin_bit_cast(bf16x8_t, w),
+                                  __builtin_bit_cast(bf16x8_t, as[16 * m + r][q * 16 + 4 * j + g]), acc[m]);
         }
       }
-    }
-    float* pp = part + (size_t)slice * M * N;
+      // weights as the first operand: lane (r, g) holds features 4g .. +3 of row 16m + r, one 16-byte store
+      if (nt * 16 >= N) return;
 #pragma unroll
-    for (int m = 0; m < 4; ++m) {
-      if (m >= mt_count) break;
-#pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        const int row = m0 + 16 * m + 4 * g + v;
-        if (row < M) pp[(size_t)row * N + feat] = acc[m][v];
+      for (int m = 0; m < MT; ++m) {
+        const int row = m0 + 16 * m + r;
+        if (row >= M) continue;
+        auto* o = reinterpret_cast<f32x4_dw*>(pp + (size_t)row * N + nt * 16 + 4 * g);
+        if (WAVES == 8) __builtin_nontemporal_store(acc[m], o);  // planes beyond L2: 137 rows 18.3 -> 16.6 us
+        else *o = acc[m];
       }
-    }
+    };
+    const int mt_count = (min(kGemmRows, M - m0) + 15) / 16;
+    if (mt_count == 4) pass(std::integral_constant<int, 4>{});
+    else if (mt_count == 3) pass(std::integral_constant<int, 3>{});
+    else if (mt_count == 2) pass(std::integral_constant<int, 2>{});
+    else pass(std::integral_constant<int, 1>{});
   }
 }
 
@@ -223,17 +191,38 @@ __device__ __forceinline__ void row_residual(const float* __restrict__ part, int
   }
 }
 
-// y = bf16(sum + b); with residual: residual <- bf16(residual + y)
+// y = bf16(sum + b); with residual: residual <- bf16(residual + y).  A thread takes four features of a row
+// (N % 16 == 0), NS the slices loaded before the first add (clamped past `slices`, never added).  It moves bytes
+// only: one feature a thread took 14.4 us for 1,024 rows of 5,120 from one plane,
+// 7.8 for 512; four take 7.0 and 4.5.
+template <int NS>
 __global__ __launch_bounds__(256) void linear_finalize_kernel(const float* __restrict__ part, int slices,
                                                               const uint16_t* __restrict__ b, int M,
                                                               int N, uint16_t* __restrict__ y,
                                                               uint16_t* __restrict__ residual) {
-  const size_t idx = (size_t)blockIdx.x * 256 + threadIdx.x;
-  if (idx >= (size_t)M * N) return;
-  const int f = idx % N;
-  const float o = bf16_round(sum_slices(part, slices, (size_t)M * N, idx) + (b ? bf2f(b[f]) : 0.f));
-  if (residual) residual[idx] = f2bf(bf2f(residual[idx]) + o);
-  else y[idx] = f2bf(o);
+  const size_t idx = ((size_t)blockIdx.x * 256 + threadIdx.x) * 4;
+  const size_t plane = (size_t)M * N;
+  if (idx >= plane) return;
+  f32x4_dw v[NS];
+#pragma unroll
+  for (int i = 0; i < NS; ++i) v[i] = *reinterpret_cast<const f32x4_dw*>(part + min(i, slices - 1) * plane + idx);
+  u16x4_h bv = {0, 0, 0, 0}, rv = {0, 0, 0, 0};
+  if (b) bv = *reinterpret_cast<const u16x4_h*>(b + idx % N);
+  if (residual) rv = *reinterpret_cast<const u16x4_h*>(residual + idx);
+  f32x4_dw o = v[0];
+#pragma unroll
+  for (int i = 1; i < NS; ++i)
+    if (i < slices) {
+#pragma unroll
+      for (int c = 0; c < 4; ++c) o[c] += v[i][c];
+    }
+  u16x4_h out;
+#pragma unroll
+  for (int c = 0; c < 4; ++c) {
+    const float r = bf16_round(o[c] + (b ? bf2f(bv[c]) : 0.f));
+    out[c] = residual ? f2bf(bf2f(rv[c]) + r) : f2bf(r);
+  }
+  *reinterpret_cast<u16x4_h*>((residual ? residual : y) + idx) = out;
 }
 
 // o_proj epilogue fused with the post-attention RMSNorm: h <- bf16(h + bf16(sum + b)),
@@ -746,8 +735,11 @@ size_t linear_partials_bytes(int M, int N, int K) { return (size_t)gemm_slices(K
 
 int launch_gemm_splitk(const uint16_t* x, const uint16_t* W, int M, int N, int K, float* part,
                        hipStream_t s) {
-  hipLaunchKernelGGL(gemm_splitk_bf16_kernel, dim3(ceil_div(N, 64), gemm_slices(K)), dim3(256), 0, s,
-                     x, W, M, N, K, part);
+  const int slices = gemm_slices(K);
+  if (M > kGemmRows)
+    hipLaunchKernelGGL(gemm_splitk_bf16_kernel<8>, dim3(ceil_div(N, 128), slices), dim3(512), 0, s, x, W, M, N, K, part);
+  else
+    hipLaunchKernelGGL(gemm_splitk_bf16_kernel<4>, dim3(ceil_div(N, 64), slices), dim3(256), 0, s, x, W, M, N, K, part);
   return check_launch("gemm_splitk_bf16");
 }
 
@@ -778,9 +770,14 @@ int launch_linear(const uint16_t* x, const uint16_t* W, const uint16_t* b, int M
   int slices = 0;
   int rc = launch_gemm(x, W, M, N, K, part, &slices, s);
   if (rc) return rc;
-  const size_t total = (size_t)M * N;
-  hipLaunchKernelGGL(linear_finalize_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, s,
-                     part, slices, b, M, N, y, residual);
+  const unsigned blocks = (unsigned)(((size_t)M * N / 4 + 255) / 256);
+  auto go = [&](auto ns) {
+    hipLaunchKernelGGL(linear_finalize_kernel<decltype(ns)::value>, dim3(blocks), dim3(256), 0, s, part, slices, b, M, N, y,
+                       residual);
+  };
+  if (slices == 1) go(std::integral_constant<int, 1>{});
+  else if (slices <= 8) go(std::integral_constant<int, 8>{});
+  else go(std::integral_constant<int, kMaxSlices>{});
   return check_launch("linear_finalize");
 }
 

@@ -300,6 +300,41 @@ def test_rmsnorm_and_linear_vs_oracle():
     assert mar < 1e-2 and cos > 0.9999
 
 
+@pytest.mark.parametrize("M", [2, 16, 17, 48, 64, 65, 80, 128, 129, 255, 256])
+@pytest.mark.parametrize("N,K,off", [(16, 32, 0), (144, 544, 1), (272, 2880, 0), (64, 8192, 3)])
+def test_linear_rows_do_not_depend_on_the_batch(M, N, K, off):
+    """Row tiles and passes of the projections: every row of a batch equals that row alone bit for bit, with
+    and without bias and residual, for N past the last whole workgroup, K of partial groups and slices, tensors
+    that start `off` elements past a 16-byte boundary, and an infinity and a NaN in the first and last rows."""
+    from flyai_amd import ops
+
+    def at(t):
+        buf = torch.empty(t.numel() + off, dtype=t.dtype, device=DEV)
+        buf[off:] = t.reshape(-1)
+        return buf[off:].view(t.shape)
+
+    x = torch.randn(M, K, device=DEV, generator=_gen(71)).to(torch.bfloat16)
+    x[0, K - 1], x[M - 1, 0] = float("inf"), float("nan")
+    w = at((torch.randn(N, K, device=DEV, generator=_gen(72)) * 0.02).to(torch.bfloat16))
+    b = at(torch.randn(N, device=DEV, generator=_gen(73)).to(torch.bfloat16))
+    res = torch.randn(M, N, device=DEV, generator=_gen(74)).to(torch.bfloat16)
+    x, res0 = at(x), at(res)
+    y = ops.linear(x, w, b)
+    y0 = ops.linear(x, w)
+    yr = ops.linear(x, w, b, residual=res0)
+    for r in sorted({0, 1, 15, 16, M // 2, 63, 64, M - 2, M - 1}):
+        if r >= M:
+            continue
+        one = at(x[r:r + 1])
+        assert torch.equal(ops.linear(one, w, b).view(torch.int16), y[r:r + 1].view(torch.int16)), r
+        assert torch.equal(ops.linear(one, w).view(torch.int16), y0[r:r + 1].view(torch.int16)), r
+        assert torch.equal(ops.linear(one, w, b, residual=at(res[r:r + 1])).view(torch.int16), yr[r:r + 1].view(torch.int16)), r
+    # fp32 sums of K exact products: K 2^-24 of the sum of magnitudes; then bf16 roundings (2^-8 each) of y
+    ref = x[1:M - 1].double() @ w.double().T + b.double()
+    mag = x[1:M - 1].double().abs() @ w.double().abs().T
+    assert bool(((y[1:M - 1].double() - ref).abs() <= K * 2.0**-24 * mag + 2.0**-8 * ref.abs() + 1e-30).all())
+
+
 @pytest.mark.parametrize("N,K", [(5120, 2880), (2880, 4096), (2000, 2880), (1008, 2080), (512, 7168)])
 def test_linear_tiled_equals_split_k_bit_exact(N, K):
     """Prefill-sized batches (>= 256 rows) take a tiled GEMM, decode-sized ones the split-K GEMM;
