@@ -76,27 +76,6 @@ __global__ __launch_bounds__(256) void mxfp4_repack_kernel(const uint8_t* __rest
 // registers (gfx950 v_cvt_scalef32_pk_bf16_fp4, E8M0 scale in the exponent field) and fed to v_mfma_f32_16x16x32_bf16 with the activation
 // fragment read from LDS (rows >= the pass's row count read as zero).  Larger groups take further
 // passes over the weights.
-typedef unsigned int u32x4_t __attribute__((ext_vector_type(4)));
-
-// Buffer resource word 3 for raw (unformatted, unswizzled) loads on gfx9, and an offset past any
-// resource this file builds (such a load returns zero and touches no memory).
-constexpr int kBufRsrcWord3 = 0x00020000;
-constexpr uint32_t kBufOutside = 0x80000000u;
-
-// A wave-uniform value, in a scalar register.  Some uniform integers (a clamp, the wave's number) come from
-// vector instructions, and a buffer resource built from one that stays in a vector register makes the
-// compiler wrap every load through it in a loop over the wave's "different" resources: a dozen
-// instructions a load, and no scheduling across it.  Decode expert kernels with and without those loops
-// (128 experts, top-4, H = I = 2880): 56 tokens 161 -> 147 us gate_up and 86 -> 80 us down, 12 tokens 63.6 ->
-// 59.9 and 39.9 -> 36.8, 200 tokens 243 -> 221 and 134 -> 127.
-__device__ __forceinline__ int scalar(int v) { return __builtin_amdgcn_readfirstlane(v); }
-
-// 16 bytes through a buffer resource, nontemporal
-__device__ __forceinline__ uint4 buf_ld16_nt(__amdgpu_buffer_rsrc_t rs, uint32_t off) {
-  const u32x4_t v = __builtin_amdgcn_raw_buffer_load_b128(rs, off, 0, 2);
-  return make_uint4(v.x, v.y, v.z, v.w);
-}
-
 __device__ __forceinline__ uint4 ld_nt(const uint8_t* p) {
   const u32x4_t v = __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(p));
   return make_uint4(v.x, v.y, v.z, v.w);

@@ -17,14 +17,9 @@ namespace flyai {
 constexpr int kTailWaves = 4;
 constexpr int kTailNTW = 2;                                   // vocab tiles per wave
 constexpr int kTailRowsPerWG = kTailWaves * kTailNTW * 16;    // 128 vocab rows per workgroup
+constexpr int kTailDepth = 8;                                 // weight ring depth, MFMA steps
+constexpr int kTailChunk = 4;                                 // MFMA steps a chunk of hidden fragments
 constexpr int kTailMaxRows = 64;                              // token rows per launch (4 tiles)
-
-typedef unsigned int tail_u32x4 __attribute__((ext_vector_type(4)));
-
-__device__ __forceinline__ uint4 tail_ld_nt(const uint8_t* p) {
-  const tail_u32x4 v = __builtin_nontemporal_load(reinterpret_cast<const tail_u32x4*>(p));
-  return make_uint4(v.x, v.y, v.z, v.w);
-}
 
 // (value desc, id asc): the first maximal index, as torch.argmax returns it
 __device__ __forceinline__ bool tail_better(float v, int i, float bv, int bi) {
@@ -60,10 +55,14 @@ __global__ __launch_bounds__(256) void embed_gather_kernel(const uint16_t* __res
 
 // ---- lm_head + argmax --------------------------------------------------------------------------
 // Workgroup = 4 waves x 2 vocab tiles = 128 vocab rows, all TT token tiles (16 token rows each).
-// K advances in chunks of 4 MFMA steps (128 K): the chunk's hidden fragments live in one of two
+// K advances in chunks of kTailChunk MFMA steps: the chunk's hidden fragments live in one of two
 // LDS buffers (TT KiB per step), the next chunk's are loaded into registers one chunk ahead, and
-// the weights go through a 4-deep register ring (3 steps in flight while one computes).  One
-// workgroup barrier per chunk.  Logits are rounded to bf16 (the reference's bf16 lm_head output)
+// the weights go through a register ring of kTailDepth steps (all but one in flight while one computes).  One
+// workgroup barrier per chunk.  The weights stream from HBM is what bounds it; their loads go through a buffer
+// resource (a tile past the last, or a step past K, reads zero with no memory access), so no branch separates a load
+// from the ring and the compiler's waits count the ring exactly.
+// 201,088 x 2,880 (1.16 GB): 1 row 208 us with predicated loads and 3 steps in flight, now 175 (6.6 TB/s); 24 rows
+// 204 -> 185, 64 rows 286 -> 228; chunks of 8 steps leave fewer workgroups a CU at 3 and 4 row tiles (219, 236).  Logits are rounded to bf16 (the reference's bf16 lm_head output)
 // and reduced to (max, lowest id) per token over the workgroup; argmax_finish_kernel folds the
 // workgroups.
 template <int TT>
@@ -71,50 +70,56 @@ __global__ __launch_bounds__(256) void lm_head_argmax_kernel(
     const uint16_t* __restrict__ x, const int32_t* __restrict__ rows, int n_rows, int K,
     const uint8_t* __restrict__ wp, int V, float* __restrict__ part_val, int32_t* __restrict__ part_id,
     uint16_t* __restrict__ logits_out) {
-  __shared__ uint4 xs[2][TT][4][64];
+  __shared__ uint4 xs[2][TT][kTailChunk][64];
   __shared__ float red_v[kTailWaves][TT * 16];
   __shared__ int red_i[kTailWaves][TT * 16];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, wave = scalar(tid >> 6);
   const int n = lane & 15, g = lane >> 4;
-  const int S = K / 32;                 // MFMA steps
-  const int NC = (S + 3) / 4;           // chunks of 4 steps
+  const int S = K / 32;                              // MFMA steps
   const int n_tiles = V / 16;
   const int t0 = (blockIdx.x * kTailWaves + wave) * kTailNTW;
 
-  // staging: thread tid covers, for each token tile tt, step j = tid/64 of the chunk, fragment lane
-  // tid%64 -> token row 16tt + (tid & 15), K 32*(4c + j) + 8*((tid & 63) >> 4)
-  const int sj = tid >> 6, sn = tid & 15, sg = (tid & 63) >> 4;
+  // staging: wave w covers, for each token tile tt, steps w, w + 4, .. of the chunk, fragment lane `lane` -> token
+  // row 16tt + n, K 32s + 8g; rows past n_rows read the last one (their logits are not stored)
+  constexpr int kXSteps = kTailChunk / kTailWaves;
   const uint16_t* srow[TT];
 #pragma unroll
   for (int tt = 0; tt < TT; ++tt) {
-    const int rr = 16 * tt + sn;
-    srow[tt] = rr < n_rows ? x + (size_t)(rows ? rows[rr] : rr) * K : nullptr;
+    const int rr = min(16 * tt + n, n_rows - 1);
+    srow[tt] = x + (size_t)(rows ? rows[rr] : rr) * K + 8 * g;
   }
-  auto load_x = [&](uint4 (&xr)[TT], int c) {
-    const int s = 4 * c + sj;
+  u32x4_t xr[TT][kXSteps];
+  auto load_x = [&](int c) __attribute__((always_inline)) {
 #pragma unroll
     for (int tt = 0; tt < TT; ++tt)
-      xr[tt] = (srow[tt] && s < S) ? *reinterpret_cast<const uint4*>(srow[tt] + 32 * s + 8 * sg)
-                                   : make_uint4(0, 0, 0, 0);
-  };
-  auto store_x = [&](const uint4 (&xr)[TT], int buf) {
 #pragma unroll
-    for (int tt = 0; tt < TT; ++tt) xs[buf][tt][sj][lane] = xr[tt];
+      for (int i = 0; i < kXSteps; ++i)
+        xr[tt][i] = *reinterpret_cast<const u32x4_t*>(srow[tt] + 32 * min(kTailChunk * c + kTailWaves * i + wave, S - 1));
+  };
+  auto store_x = [&](int c) __attribute__((always_inline)) {
+#pragma unroll
+    for (int tt = 0; tt < TT; ++tt)
+#pragma unroll
+      for (int i = 0; i < kXSteps; ++i) {
+        const bool in = kTailChunk * c + kTailWaves * i + wave < S;
+        *reinterpret_cast<u32x4_t*>(&xs[c & 1][tt][kTailWaves * i + wave][lane]) = in ? xr[tt][i] : u32x4_t{0u, 0u, 0u, 0u};
+      }
   };
 
-  const uint8_t* wbase = wp + (size_t)t0 * S * 1024 + lane * 16;
-  auto load_w = [&](uint4 (&w)[kTailNTW], int s) {
+  const int ntw = scalar(max(0, min(kTailNTW, n_tiles - t0)));
+  const __amdgpu_buffer_rsrc_t wrs = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<uint8_t*>(wp + (size_t)t0 * S * 1024), (short)0, ntw * S * 1024, kBufRsrcWord3);
+  auto load_w = [&](uint4 (&w)[kTailNTW], int s) __attribute__((always_inline)) {
 #pragma unroll
     for (int nn = 0; nn < kTailNTW; ++nn)
-      w[nn] = (t0 + nn < n_tiles && s < S) ? tail_ld_nt(wbase + ((size_t)nn * S + s) * 1024)
-                                            : make_uint4(0, 0, 0, 0);
+      w[nn] = buf_ld16_nt(wrs, s < S ? (uint32_t)((nn * S + s) * 1024 + lane * 16) : kBufOutside);
   };
   f32x4_t acc[kTailNTW][TT];
 #pragma unroll
   for (int nn = 0; nn < kTailNTW; ++nn)
 #pragma unroll
     for (int tt = 0; tt < TT; ++tt) acc[nn][tt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  auto compute = [&](const uint4 (&w)[kTailNTW], int buf, int j) {
+  auto compute = [&](const uint4 (&w)[kTailNTW], int buf, int j) __attribute__((always_inline)) {
 #pragma unroll
     for (int tt = 0; tt < TT; ++tt) {
       const bf16x8_t b = as_bf16x8(xs[buf][tt][j][lane]);
@@ -123,30 +128,29 @@ __global__ __launch_bounds__(256) void lm_head_argmax_kernel(
     }
   };
 
-  uint4 xr[TT];
-  load_x(xr, 0);
-  store_x(xr, 0);
-  load_x(xr, 1);
-  uint4 w0[kTailNTW], w1[kTailNTW], w2[kTailNTW], w3[kTailNTW];
-  load_w(w0, 0);
-  load_w(w1, 1);
-  load_w(w2, 2);
+  load_x(0);
+  uint4 w[kTailDepth][kTailNTW];
+#pragma unroll
+  for (int j = 0; j < kTailDepth - 1; ++j) load_w(w[j], j);
+  store_x(0);
+  load_x(1);
   lds_barrier();
-  for (int c = 0; c < NC; ++c) {
-    const int buf = c & 1, s0 = 4 * c;
-    load_w(w3, s0 + 3);
-    compute(w0, buf, 0);
-    load_w(w0, s0 + 4);
-    compute(w1, buf, 1);
-    load_w(w1, s0 + 5);
-    compute(w2, buf, 2);
-    load_w(w2, s0 + 6);
-    compute(w3, buf, 3);
-    // the next chunk's fragments go to the other buffer: every wave finished reading it before the
-    // previous barrier, and the barrier below publishes it
-    store_x(xr, buf ^ 1);
-    load_x(xr, c + 2);
-    lds_barrier();
+  for (int s0 = 0; s0 < S; s0 += kTailDepth) {
+#pragma unroll
+    for (int h = 0; h < kTailDepth / kTailChunk; ++h) {
+      const int c = s0 / kTailChunk + h;
+#pragma unroll
+      for (int i = 0; i < kTailChunk; ++i) {
+        const int j = kTailChunk * h + i;
+        load_w(w[(j + kTailDepth - 1) % kTailDepth], s0 + j + kTailDepth - 1);
+        compute(w[j], c & 1, i);
+      }
+      // the next chunk's fragments go to the other buffer: every wave finished reading it before the
+      // previous barrier, and the barrier below publishes it
+      store_x(c + 1);
+      load_x(c + 2);
+      lds_barrier();
+    }
   }
 
   // lane (n, g) holds the logits of vocab rows 16(t0+nn) + 4g + v for token row 16tt + n

@@ -799,3 +799,29 @@ def test_medium_group_experts_bit_identical(H, I):
         h, y = run(rows)
         assert torch.equal(h.view(torch.int16), h_all[rows].view(torch.int16)), "gate_up differs"
         assert torch.equal(y.view(torch.int32), y_all[rows].view(torch.int32)), "down differs"
+
+
+@pytest.mark.parametrize("H", [32, 128, 160, 288, 2880])
+@pytest.mark.parametrize("n,V", [(1, 16), (16, 144), (17, 272), (48, 128), (64, 1040)])
+def test_lm_head_rows_do_not_depend_on_the_batch(n, V, H):
+    """K shorter than the weight ring and of partial chunks, vocabularies past the last whole workgroup, 1 to 4
+    row tiles, rows picked in any order, an infinite hidden value: every row's logits equal that row's alone bit
+    for bit and the token is their first maximum; finite rows against float64."""
+    from flyai_amd import ops
+    x = torch.randn(n + 3, H, device=DEV, generator=_gen(91)).to(torch.bfloat16)
+    w = (torch.randn(V, H, device=DEV, generator=_gen(92)) * 0.05).to(torch.bfloat16)
+    rows = torch.randperm(n + 3, generator=torch.Generator().manual_seed(n))[:n].to(torch.int32).to(DEV)
+    x[int(rows[0]), H - 1] = float("inf")
+    wp = ops.bf16_tile_repack(w)
+    ids, logits = ops.lm_head_argmax(x, wp, V, rows=rows, want_logits=True)
+    for i in sorted({0, 1, 15, 16, n - 1}):
+        if i < n:
+            i1, l1 = ops.lm_head_argmax(x, wp, V, rows=rows[i:i + 1].contiguous(), want_logits=True)
+            assert torch.equal(l1.view(torch.int16), logits[i:i + 1].view(torch.int16)) and int(i1[0]) == int(ids[i])
+    best = logits.float().amax(1, keepdim=True)
+    first = (logits.float() == best).int().argmax(1)
+    assert torch.equal(first[1:].cpu().int(), ids[1:].cpu().int())
+    # fp32 sums of H exact products: H 2^-24 of the sum of magnitudes; then one bf16 rounding (2^-8)
+    xs = x[rows.long()][1:].double()
+    ref, mag = xs @ w.double().T, xs.abs() @ w.double().abs().T
+    assert bool(((logits[1:].double() - ref).abs() <= H * 2.0**-24 * mag + 2.0**-8 * ref.abs() + 1e-30).all())
