@@ -373,40 +373,39 @@ int launch_moe_fp8(const uint8_t* aq, const uint8_t* as, const int32_t* perm, co
 }
 
 // ---- combine: out[t] = bf16(residual + bf16(sum_s y[inv[t*k+s]] + shared[t])) ------------------------
+// A thread takes four features of one token; the k rows' loads go out together (a slot past k reads the last one
+// and is not added).  It moves bytes only: with one workgroup a token and one load after the other, 155 tokens of
+// 7,168 x 8 took 26 us, now 6.3.
 __global__ __launch_bounds__(256) void moe_combine_sum_kernel(const uint16_t* __restrict__ y,
                                                               const int32_t* __restrict__ inv, int k,
                                                               int H, const uint16_t* __restrict__ shared,
                                                               const uint16_t* residual, uint16_t* out) {
   const int t = blockIdx.x;
-  int rows[8];
-  for (int s = 0; s < k; ++s) rows[s] = inv[t * k + s];
-  for (int i = threadIdx.x; i < H / 4; i += 256) {
-    float acc[4] = {0.f, 0.f, 0.f, 0.f};
-    for (int s = 0; s < k; ++s) {
-      const uint2 v = reinterpret_cast<const uint2*>(y + (size_t)rows[s] * H)[i];
-      acc[0] += bf2f(v.x & 0xffff); acc[1] += bf2f(v.x >> 16);
-      acc[2] += bf2f(v.y & 0xffff); acc[3] += bf2f(v.y >> 16);
-    }
-    if (shared) {
-      const uint2 v = reinterpret_cast<const uint2*>(shared + (size_t)t * H)[i];
-      acc[0] += bf2f(v.x & 0xffff); acc[1] += bf2f(v.x >> 16);
-      acc[2] += bf2f(v.y & 0xffff); acc[3] += bf2f(v.y >> 16);
-    }
-    uint16_t o[4];
-    if (residual) {
-      const uint2 v = reinterpret_cast<const uint2*>(residual + (size_t)t * H)[i];
-      const float rv[4] = {bf2f(v.x & 0xffff), bf2f(v.x >> 16), bf2f(v.y & 0xffff), bf2f(v.y >> 16)};
+  const int i = blockIdx.y * 256 + threadIdx.x;
+  if (i >= H / 4) return;
+  uint2 v[8], sv = make_uint2(0, 0), rv = make_uint2(0, 0);
 #pragma unroll
-      for (int c = 0; c < 4; ++c) o[c] = f2bf(rv[c] + bf16_round(acc[c]));
-    } else {
+  for (int s = 0; s < 8; ++s) v[s] = reinterpret_cast<const uint2*>(y + (size_t)inv[t * k + min(s, k - 1)] * H)[i];
+  if (shared) sv = reinterpret_cast<const uint2*>(shared + (size_t)t * H)[i];
+  if (residual) rv = reinterpret_cast<const uint2*>(residual + (size_t)t * H)[i];
+  float acc[4] = {0.f, 0.f, 0.f, 0.f};
+  auto add = [&](const uint2& u) {
+    acc[0] += bf2f(u.x & 0xffff); acc[1] += bf2f(u.x >> 16);
+    acc[2] += bf2f(u.y & 0xffff); acc[3] += bf2f(u.y >> 16);
+  };
 #pragma unroll
-      for (int c = 0; c < 4; ++c) o[c] = f2bf(acc[c]);
-    }
-    uint2 ov;
-    ov.x = (uint32_t)o[0] | ((uint32_t)o[1] << 16);
-    ov.y = (uint32_t)o[2] | ((uint32_t)o[3] << 16);
-    reinterpret_cast<uint2*>(out + (size_t)t * H)[i] = ov;
+  for (int s = 0; s < 8; ++s)
+    if (s < k) add(v[s]);
+  if (shared) add(sv);
+  if (residual) {
+    const float rf[4] = {bf2f(rv.x & 0xffff), bf2f(rv.x >> 16), bf2f(rv.y & 0xffff), bf2f(rv.y >> 16)};
+#pragma unroll
+    for (int c = 0; c < 4; ++c) acc[c] = rf[c] + bf16_round(acc[c]);
   }
+  uint2 ov;
+  ov.x = (uint32_t)f2bf(acc[0]) | ((uint32_t)f2bf(acc[1]) << 16);
+  ov.y = (uint32_t)f2bf(acc[2]) | ((uint32_t)f2bf(acc[3]) << 16);
+  reinterpret_cast<uint2*>(out + (size_t)t * H)[i] = ov;
 }
 
 }  // namespace flyai
@@ -468,7 +467,7 @@ extern "C" int flyai_moe_combine_sum(const uint16_t* y_perm, const int32_t* inv,
   FLYAI_REQUIRE(T >= 0 && k >= 1 && k <= 8 && H > 0 && H % 4 == 0, "combine_sum: bad shape");
   FLYAI_REQUIRE(y_perm && inv && out, "combine_sum: null pointer");
   if (T == 0) return FLYAI_OK;
-  hipLaunchKernelGGL(moe_combine_sum_kernel, dim3(T), dim3(256), 0, as_stream(stream), y_perm, inv, k, H,
+  hipLaunchKernelGGL(moe_combine_sum_kernel, dim3(T, ceil_div(H / 4, 256)), dim3(256), 0, as_stream(stream), y_perm, inv, k, H,
                      shared, residual, out);
   return check_launch("moe_combine_sum");
 }
