@@ -391,7 +391,12 @@ int launch_router_grouped(const uint16_t* x, const uint16_t* w, const float* e_b
   if (H <= 3072)
     hipLaunchKernelGGL((router_logits_kernel<8, 2, 6, false>), dim3(ceil_div(T, 8), ceil_div(E, 8)),
                        dim3(256), 8 * H * sizeof(uint16_t), s, x, w, nullptr, T, H, E, logits);
-  else
+  else if (ceil_div(T, 4) * ceil_div(E, 4) > 512)
+    // more workgroups than the chip holds at once (two a CU): two experts a wave share the unpacked activations,
+    // 155 tokens x 256 experts x 7,168 in 31 us where one expert a wave takes 40 (four: 39, one wave a SIMD)
+    hipLaunchKernelGGL((router_logits_kernel<4, 2, 14, false>), dim3(ceil_div(T, 4), ceil_div(E, 8)),
+                       dim3(256), 4 * H * sizeof(uint16_t), s, x, w, nullptr, T, H, E, logits);
+  else  // fewer: twice the workgroups, each half as long
     hipLaunchKernelGGL((router_logits_kernel<4, 1, 14, false>), dim3(ceil_div(T, 4), ceil_div(E, 4)),
                        dim3(256), 4 * H * sizeof(uint16_t), s, x, w, nullptr, T, H, E, logits);
   int rc = check_launch("router_logits(fp32)");

@@ -89,6 +89,22 @@ def test_grouped_router_bit_exact(T, H, E, ng, tg, k):
     assert np.array_equal(wts.cpu().numpy(), rwts)
 
 
+@pytest.mark.parametrize("T,H,E,k", [(32, 7168, 256, 8), (33, 7168, 256, 8), (66, 3592, 252, 6), (155, 4096, 64, 4)])
+def test_grouped_router_wide_rows_bit_exact(T, H, E, k):
+    """Wide rows on both sides of the two-experts-a-wave rule: the last launch below it and the first above,
+    partial token and expert groups, a partial last chunk."""
+    from flyai_amd import ops
+    g = _gen(5)
+    x = torch.randn(T, H, device=DEV, generator=g).to(torch.bfloat16)
+    w = (torch.randn(E, H, device=DEV, generator=g) * 0.02).to(torch.bfloat16)
+    ids, wts, logits = ops.router_grouped_sigmoid(x, w, None, 1, 1, k, 2.5)
+    rl = oroute.dot_fixed(x.float().cpu(), w.float().cpu()).numpy()
+    assert np.array_equal(logits.cpu().numpy(), rl)
+    rids, rwts, _ = oroute.grouped_sigmoid_route(x.float().cpu().numpy(), w.float().cpu().numpy(),
+                                                 np.zeros(E, np.float32), 1, 1, k, 2.5)
+    assert np.array_equal(ids.cpu().numpy(), rids) and np.array_equal(wts.cpu().numpy(), rwts)
+
+
 def test_grouped_router_ties_go_to_lower_ids():
     """Zero router weights make every score sigmoid(0) = 0.5; a bias with repeated values then
     leaves ties in both the group scores and the expert choices."""
