@@ -7,7 +7,7 @@ probability vector), ``uniform``, ``sample_logits`` (greedy argmax or one sample
 p_j(d_j), on the first rejection a draw from p_j with d_j removed, a bonus draw from p_K when all K
 accept; greedy -> the argmax of every row).
 
-The filtering and the draws run in ``flyai_sample_rows`` / ``flyai_sample_probs`` on the GPU over exact
+The filtering and the draws run in ``flyai_sample_rows_ws`` / ``flyai_sample_probs`` on the GPU over exact
 integer weights w = floor(2^40 e^(z - max z)); only the uniforms come from the host: a numpy PCG64
 generator seeded with ``seed``, so a run's receipts are reproducible (the reference seeds a torch
 generator instead; its stream cannot be matched, and the distribution of every output is what the
