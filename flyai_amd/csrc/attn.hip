@@ -702,18 +702,27 @@ __global__ __launch_bounds__(64, 1) void attn_tree_kernel(
                        tv);
 }
 
-// Blocks a wave of a super-block, for items of one and of two row tiles (two spill with two row tiles), and
-// the most blocks an item may have to be left to one wave, which needs no barrier: 32 windowed
-// single-token rows (3 blocks) 7.0 us by one wave, 7.6 by four; 8 windowed 4-token rows 7.8 and 6.8 us.
+// Blocks a wave of a super-block, for items of one and of two row tiles (two spill with two row tiles).
 constexpr int kCoopNB1 = 2, kCoopNB2 = 1;
-constexpr int kSoloBlocks1 = 3, kSoloBlocks2 = 1;
+
+// The most blocks an item may have to be left to one wave, which needs no barrier.  One wave / four waves an
+// item, us:
+//   1 token, 32 windowed rows (3 blocks) 7.0 / 7.6, 64 items of 4 blocks 8.1 / 7.6; 2 tokens, 256 items of 4
+//   blocks 8.7 / 9.1, of 5 blocks 9.4 / 9.0 (a wave with one token masks the unused half of its row tile in every
+//   block: four waves share that);
+//   more workgroups than CUs, 512 items: 1 token, 4 blocks 10.0 / 11.0, 6 blocks 13.2 / 12.2; 2 tokens, 4 blocks
+//   9.3 / 11.3, 6 blocks 12.3 / 12.2;
+//   4 tokens (two row tiles): 2 blocks, 64 items 7.5 / 7.6, 512 items 8.2 / 9.4; 3 blocks, 64 items 8.8 / 7.8; 4
+//   blocks, 512 items 12.1 / 11.0.
+constexpr int kSoloBlocks2 = 2;
+__device__ __forceinline__ int solo_blocks(int ntok, int full) { return ntok > 2 ? kSoloBlocks2 : full ? 5 : ntok == 2 ? 4 : 3; }
 
 union CoopAny {
   CoopShared<1, kCoopNB1> one;
   CoopShared<2, kCoopNB2> two;
 };
 
-template <int QT, bool TREE, int NB, int SOLO>
+template <int QT, bool TREE, int NB>
 __device__ __forceinline__ void attn_item_any(const flyai_attn_item& it, const uint16_t* __restrict__ q,
                                               const uint16_t* __restrict__ k_pool,
                                               const uint16_t* __restrict__ v_pool,
@@ -722,8 +731,8 @@ __device__ __forceinline__ void attn_item_any(const flyai_attn_item& it, const u
                                               float* __restrict__ partials,
                                               const flyai_attn_group* __restrict__ groups, int n_groups,
                                               const float* __restrict__ sinks, uint16_t* __restrict__ out,
-                                              const TreeView& tv, CoopShared<QT, NB>& sh) {
-  if (it.key_hi - (it.key_lo & ~63) > 64 * SOLO)
+                                              const TreeView& tv, CoopShared<QT, NB>& sh, int solo) {
+  if (it.key_hi - (it.key_lo & ~63) > 64 * solo)
     attn_item_coop<QT, TREE, NB>(it, blockIdx.x, q, k_pool, v_pool, kv_base, kv_cap, window, Hq, partials, groups,
                                  n_groups, sinks, out, tv, sh);
   else if (threadIdx.x < 64)
@@ -731,23 +740,25 @@ __device__ __forceinline__ void attn_item_any(const flyai_attn_item& it, const u
                         sinks, out, tv);
 }
 
-// attn_partial_kernel and attn_tree_kernel with a workgroup of kCoopWaves waves an item
+// attn_partial_kernel and attn_tree_kernel with a workgroup of kCoopWaves waves an item.  full: the launch has
+// more workgroups than CUs.
 __global__ __launch_bounds__(64 * kCoopWaves, 2) void attn_coop_kernel(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ k_pool,
     const uint16_t* __restrict__ v_pool, const int64_t* __restrict__ kv_base,
     const int32_t* __restrict__ kv_cap, int window, int Hq,
     const flyai_attn_item* __restrict__ items, const int32_t* __restrict__ n_live,
     float* __restrict__ partials, const flyai_attn_group* __restrict__ groups, int n_groups,
-    const float* __restrict__ sinks, uint16_t* __restrict__ out) {
+    const float* __restrict__ sinks, uint16_t* __restrict__ out, int full) {
   __shared__ CoopAny sh;
   if (n_live && (int)blockIdx.x >= *n_live) return;  // as in attn_partial_kernel
   const flyai_attn_item it = items[blockIdx.x];
+  const int solo = solo_blocks(it.ntok, full);
   if (it.ntok <= 2)
-    attn_item_any<1, false, kCoopNB1, kSoloBlocks1>(it, q, k_pool, v_pool, kv_base, kv_cap, window, Hq, partials, groups,
-                                                    n_groups, sinks, out, TreeView{}, sh.one);
+    attn_item_any<1, false, kCoopNB1>(it, q, k_pool, v_pool, kv_base, kv_cap, window, Hq, partials, groups,
+                                      n_groups, sinks, out, TreeView{}, sh.one, solo);
   else
-    attn_item_any<2, false, kCoopNB2, kSoloBlocks2>(it, q, k_pool, v_pool, kv_base, kv_cap, window, Hq, partials, groups,
-                                                    n_groups, sinks, out, TreeView{}, sh.two);
+    attn_item_any<2, false, kCoopNB2>(it, q, k_pool, v_pool, kv_base, kv_cap, window, Hq, partials, groups,
+                                      n_groups, sinks, out, TreeView{}, sh.two, solo);
 }
 
 __global__ __launch_bounds__(64 * kCoopWaves, 1) void attn_tree_coop_kernel(
@@ -760,12 +771,13 @@ __global__ __launch_bounds__(64 * kCoopWaves, 1) void attn_tree_coop_kernel(
   __shared__ CoopAny sh;
   const flyai_attn_item it = items[blockIdx.x];
   const TreeView tv = tree_view(tree, window);
+  const int solo = solo_blocks(it.ntok, 0);
   if (it.ntok <= 2)
-    attn_item_any<1, true, kCoopNB1, kSoloBlocks1>(it, q, k_pool, v_pool, kv_base, kv_cap, window, Hq, partials, groups,
-                                                   n_groups, sinks, out, tv, sh.one);
+    attn_item_any<1, true, kCoopNB1>(it, q, k_pool, v_pool, kv_base, kv_cap, window, Hq, partials, groups,
+                                     n_groups, sinks, out, tv, sh.one, solo);
   else
-    attn_item_any<2, true, kCoopNB2, kSoloBlocks2>(it, q, k_pool, v_pool, kv_base, kv_cap, window, Hq, partials, groups,
-                                                   n_groups, sinks, out, tv, sh.two);
+    attn_item_any<2, true, kCoopNB2>(it, q, k_pool, v_pool, kv_base, kv_cap, window, Hq, partials, groups,
+                                     n_groups, sinks, out, tv, sh.two, solo);
 }
 
 // ---- chunked-prefill rows -------------------------------------------------------------------------
@@ -1027,11 +1039,13 @@ __global__ __launch_bounds__(256) void attn_merge_kernel(const float* __restrict
   *reinterpret_cast<uint4*>(o) = make_uint4(wv[0], wv[1], wv[2], wv[3]);
 }
 
-// Up to this many items a workgroup of four waves takes each; past it the chip is full with one wave an item
-// and the barriers only cost.  One wave / four waves an item, items of up to 16 blocks: 16 items 16.0 /
-// 9.3 us, 128 24.7 / 15.1, 248 25.2 / 16.7, 384 27.4 / 21.2, 544 34.1 / 30.3, 880 39.8 / 41.1,
-// 1264 48.8 / 52.7.
-constexpr int kCoopItems = 640;
+// Four waves take an item while all the launch's workgroups are on the chip at once: two a CU of the decode kernel
+// (249 registers a wave), one of the tree kernel (336).  Past that the workgroups queue behind one another, where
+// one wave an item (8 and 4 items a CU at once) still has its turn.  One wave / four waves an item, items of 16 blocks
+// of one token: 16 items 16.0 / 9.3 us, 128 24.7 / 15.1, 256 25.8 / 17.0, 512 30.3 / 26.1, 640 32.1 / 34.7; of four tokens
+// and 2 blocks, 640 items: 8.6 / 12.3.  Trees over 8,000 keys: 18 nodes (320 items) 25.9 / 32.6 us, 32 nodes (512 items)
+// 28.5 / 36.8; over 3,000 keys 32 nodes (192 items) 33.1 / 20.8.
+inline int coop_items(bool tree) { return (tree ? 1 : 2) * device_cus(); }
 
 // n_items / n_groups size the grids; counts (nullable) holds this step's live item and group
 // counts on the device, for launches sized by a plan capacity (graph replay)
@@ -1042,7 +1056,7 @@ int launch_attn(const uint16_t* q, const uint16_t* k_pool, const uint16_t* v_poo
                 uint16_t* out, const flyai_attn_tree* tree, bool merge, hipStream_t s) {
   if (n_items == 0) return FLYAI_OK;
   (void)n_small;  // the plan's two ranges share one launch
-  const bool coop = n_items <= kCoopItems;
+  const bool coop = n_items <= coop_items(tree != nullptr);
   if (tree && coop)  // a tree is launched directly with exact counts (never from a graph)
     hipLaunchKernelGGL(attn_tree_coop_kernel, dim3(n_items), dim3(64 * kCoopWaves), 0, s, q, k_pool, v_pool, kv_base,
                        kv_cap, window, Hq, items, partials, groups, n_groups, sinks, out, tree);
@@ -1051,7 +1065,7 @@ int launch_attn(const uint16_t* q, const uint16_t* k_pool, const uint16_t* v_poo
                        Hq, items, partials, groups, n_groups, sinks, out, tree);
   else if (coop)
     hipLaunchKernelGGL(attn_coop_kernel, dim3(n_items), dim3(64 * kCoopWaves), 0, s, q, k_pool, v_pool, kv_base,
-                       kv_cap, window, Hq, items, counts, partials, groups, n_groups, sinks, out);
+                       kv_cap, window, Hq, items, counts, partials, groups, n_groups, sinks, out, n_items > device_cus());
   else
     hipLaunchKernelGGL(attn_partial_kernel, dim3(n_items), dim3(64), 0, s, q, k_pool, v_pool, kv_base,
                        kv_cap, window, Hq, items, counts, partials, groups, n_groups, sinks, out);

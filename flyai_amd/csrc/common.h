@@ -4,6 +4,8 @@
 #include <stdint.h>
 #include <stddef.h>
 
+#include <atomic>
+
 #include "flyai_stage.h"
 
 namespace flyai {
@@ -227,6 +229,19 @@ __device__ __forceinline__ uint4 buf_ld16_nt(__amdgpu_buffer_rsrc_t rs, uint32_t
 }
 
 inline hipStream_t as_stream(flyai_stream_t s) { return reinterpret_cast<hipStream_t>(s); }
+
+// CUs of the device current at the call (read once per device).
+inline int device_cus() {
+  constexpr int kDevices = 64;
+  static std::atomic<int> cached[kDevices];
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kDevices) return 256;
+  int v = cached[dev].load(std::memory_order_relaxed);
+  if (v > 0) return v;
+  if (hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || v <= 0) v = 256;
+  cached[dev].store(v, std::memory_order_relaxed);
+  return v;
+}
 
 inline int ceil_div(int a, int b) { return (a + b - 1) / b; }
 

@@ -14,7 +14,6 @@
 // 32*(4kg+g) + 8j .. +7 for BOTH operands: the lane's 16 weight bytes feed four MFMA steps and
 // its activation bytes are the matching 64 contiguous bytes of the activation row.
 #include <algorithm>
-#include <atomic>
 #include <type_traits>
 
 #include "common.h"
@@ -1181,19 +1180,6 @@ __global__ __launch_bounds__(512) void moe_mx_gemm_kernel(
 // Chunk of weight blocks per workgroup: the largest chunk that still gives at least 3 rounds of
 // workgroups over the CUs, so that workgroups of unequal length (experts with different row
 // counts take different row tiles) balance, while each start-up is shared by several blocks.
-// The CU count is read per device (once each) for the device current at the call.
-inline int device_cus() {
-  constexpr int kDevices = 64;
-  static std::atomic<int> cached[kDevices];
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kDevices) return 256;
-  int v = cached[dev].load(std::memory_order_relaxed);
-  if (v > 0) return v;
-  if (hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || v <= 0) v = 256;
-  cached[dev].store(v, std::memory_order_relaxed);
-  return v;
-}
-
 inline int gemm_chunk(const MxGeom& gm, int E) {
   const int cus = device_cus();
   const int W = (gm.NT + kGemmTiles - 1) / kGemmTiles;

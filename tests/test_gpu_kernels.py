@@ -526,6 +526,43 @@ def test_attention_few_items_equal_many_items_bit_exact(window, split):
     assert torch.isfinite(many.float()).all()
 
 
+@pytest.mark.parametrize("window", [0, 128])
+@pytest.mark.parametrize("q_len", [1, 2, 4])
+def test_attention_item_count_rules_bit_exact(q_len, window):
+    """The launch's item count decides how many waves take an item and up to how many blocks one wave takes it
+    alone (one workgroup a CU, two a CU, more): the same sequences in launches on both sides of every line, with
+    key counts at both sides of every block line, give the same bits."""
+    from flyai_amd import ops
+    Hq, Hkv, D, cap, S = 64, 8, 64, 640, 72
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    starts = [(64 * (1 + b % 9) + (b % 5) - 2) - q_len for b in range(S)]
+    slab = Hkv * cap * D
+    kp = torch.full((S * slab,), float("nan"), device=DEV, dtype=torch.bfloat16)
+    vp = torch.full((S * slab,), float("nan"), device=DEV, dtype=torch.bfloat16)
+    for b, st in enumerate(starts):
+        pos = torch.arange(st + q_len, device=DEV)
+        kvlayout.scatter(kp[b * slab:(b + 1) * slab], Hkv, cap, "k",
+                         4 * torch.randn(Hkv, st + q_len, D, device=DEV, generator=_gen(700 + b)), pos)
+        kvlayout.scatter(vp[b * slab:(b + 1) * slab], Hkv, cap, "v",
+                         torch.randn(Hkv, st + q_len, D, device=DEV, generator=_gen(800 + b)), pos)
+    q = (4 * torch.randn(S * q_len, Hq, D, device=DEV, generator=_gen(56))).to(torch.bfloat16)
+    sinks = torch.randn(Hq, device=DEV, generator=_gen(57)).to(torch.bfloat16).float()
+
+    def run(n):
+        base = torch.arange(n, dtype=torch.int64, device=DEV) * slab
+        capt = torch.full((n,), cap, dtype=torch.int32, device=DEV)
+        items, groups, n_small = ops.attn_plan([q_len] * n, starts[:n], Hkv, window, 1024)
+        out = ops.attn_ragged(q[:n * q_len].contiguous(), kp, vp, base, capt, sinks, window, items, groups, n_small, Hkv)
+        return out.view(torch.int16), len(items)
+
+    many, n_many = run(S)
+    assert n_many > 2 * cus and torch.isfinite(many.view(torch.bfloat16).float()).all()
+    for n in (1, cus // 8, cus // 8 + 1, cus // 4, cus // 4 + 1):
+        few, n_items = run(n)
+        assert n_items == 8 * n
+        assert torch.equal(few, many[:n * q_len]), n
+
+
 def test_attention_ignores_unwritten_nan_slots():
     """Keys/values past each sequence's length (and before its window) are never read into the
     result even when they hold NaN: the kernel masks scores and zeroes out-of-range values."""
