@@ -38,9 +38,9 @@ constexpr int kGemmRows = 64; // activation rows per pass
 // are loaded into registers under the current pass's MFMAs (one barrier pair a pass, on LDS only: the loads stay in
 // flight).  A pass used to be staged behind a barrier that drained every load, by workgroups of 64 features: the
 // two projections of 5,120 x 2,880 and 2,880 x 4,096 took 19.2 and 18.5 us at 137 rows, now 16.3 and 15.6; 24.9 and
-// 24.3 at 255, now 22.5 and 22.2.  Eight waves and 128 features read the activations half as often from L2; wider
-// waves (two feature tiles each) made no difference.  What is left past the weights' 5 us is the partial planes'
-// way out, about 4 us per 64 rows, which the slice order of the sums needs.
+// 24.3 at 255, now 22.5 and 22.2.  Eight waves and 128 features read the activations half as often from L2, where
+// that grid still gives most CUs a workgroup (launch_gemm_splitk); wider waves (two feature tiles each) made no
+// difference.  What is left past the weights' 5 us is the partial planes' way out, about 4 us per 64 rows.
 // No load sits under a lane's branch: rows past M and features past N read a clamped one (their sums are not
 // stored), K past the row's end is replaced by zero in both operands.  With the loads predicated the weights' waited
 // for the activations' to return: 7.7 us for 1 row of either projection, 8.1 for 16; now 7.2 and 7.5.
@@ -736,7 +736,14 @@ size_t linear_partials_bytes(int M, int N, int K) { return (size_t)gemm_slices(K
 int launch_gemm_splitk(const uint16_t* x, const uint16_t* W, int M, int N, int K, float* part,
                        hipStream_t s) {
   const int slices = gemm_slices(K);
-  if (M > kGemmRows)
+  // Past 64 rows eight waves and 128 features a workgroup, where those workgroups have a CU each and those of four waves
+  // would not.  With fewer, half of the chip is idle; with more, the second round is as long as the first.  Kernel and
+  // finalize at 137 rows, four waves / eight: 512 x 512 (4 workgroups of eight waves) 11.0 / 15.0 us, 1,024 x 2,880
+  // (48) 13.3 / 17.0, 2,048 x 2,880 (96) 15.4 / 18.0, 1,024 x 8,192 (128) 16.2 / 19.0; 2,880 x 2,880 (138) 19.1 / 18.4,
+  // 2,880 x 4,096 (184) 20.7 / 19.3, 5,120 x 2,880 (240) 22.6 / 20.8; 5,120 x 4,608 (360) 32.0 / 34.3, 2,880 x 8,192
+  // (368) 32.4 / 35.5.
+  const int cus = device_cus();
+  if (M > kGemmRows && (int64_t)ceil_div(N, 64) * slices > cus && (int64_t)ceil_div(N, 128) * slices <= cus)
     hipLaunchKernelGGL(gemm_splitk_bf16_kernel<8>, dim3(ceil_div(N, 128), slices), dim3(512), 0, s, x, W, M, N, K, part);
   else
     hipLaunchKernelGGL(gemm_splitk_bf16_kernel<4>, dim3(ceil_div(N, 64), slices), dim3(256), 0, s, x, W, M, N, K, part);

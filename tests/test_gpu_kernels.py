@@ -335,6 +335,28 @@ def test_linear_rows_do_not_depend_on_the_batch(M, N, K, off):
     assert bool(((y[1:M - 1].double() - ref).abs() <= K * 2.0**-24 * mag + 2.0**-8 * ref.abs() + 1e-30).all())
 
 
+# grids of eight waves a workgroup (the first), and of four on both sides of them
+@pytest.mark.parametrize("M", [65, 128, 137, 255])
+@pytest.mark.parametrize("N,K,off", [(2896, 2880, 1), (1040, 2880, 0), (5136, 4608, 0), (272, 512, 3)])
+def test_linear_passes_of_64_rows_bit_exact(M, N, K, off):
+    """Batches of several passes by workgroups of four and of eight waves: every tile's first and last row equals
+    that row alone bit for bit (a last workgroup with tiles past N, a last slice of fewer groups than the others)."""
+    from flyai_amd import ops
+
+    def at(t):
+        buf = torch.empty(t.numel() + off, dtype=t.dtype, device=DEV)
+        buf[off:] = t.reshape(-1)
+        return buf[off:].view(t.shape)
+
+    x = torch.randn(M, K, device=DEV, generator=_gen(75)).to(torch.bfloat16)
+    x[M - 1, 0] = float("nan")
+    w = at((torch.randn(N, K, device=DEV, generator=_gen(76)) * 0.02).to(torch.bfloat16))
+    b = at(torch.randn(N, device=DEV, generator=_gen(77)).to(torch.bfloat16))
+    y = ops.linear(at(x), w, b)
+    for r in sorted({r for m in range(0, M, 16) for r in (m, min(m + 15, M - 1))}):
+        assert torch.equal(ops.linear(at(x[r:r + 1]), w, b).view(torch.int16), y[r:r + 1].view(torch.int16)), r
+
+
 @pytest.mark.parametrize("N,K", [(5120, 2880), (2880, 4096), (2000, 2880), (1008, 2080), (512, 7168)])
 def test_linear_tiled_equals_split_k_bit_exact(N, K):
     """Prefill-sized batches (>= 256 rows) take a tiled GEMM, decode-sized ones the split-K GEMM;
