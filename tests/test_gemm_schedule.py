@@ -135,3 +135,19 @@ def test_medium_kernel_groups(gemm_asm_mid):
             bounds = waits + [hi]
             for a, b in zip(bounds, bounds[1:]):
                 assert Counter(_ops(body[a:b])) == _group(1), f"{name}: group issue {_ops(body[a:b])}"
+
+
+def test_projection_activations_do_not_wait_for_the_weights(tmp_path):
+    """gemm_splitk_bf16_kernel issues the activation loads, then its 16 weight loads, and stores the activations to
+    LDS: the first store's wait must leave the weight loads in flight (vector-memory loads complete in order)."""
+    out = tmp_path / "linear.s"
+    flags = [f for f in B.FLAGS if f != "-fPIC"]
+    r = subprocess.run([HIPCC, *flags, "-S", "--cuda-device-only", "-x", "hip", os.path.join(B.CSRC, "linear.hip"), "-o", str(out)],
+                       capture_output=True, text=True)
+    assert r.returncode == 0, r.stderr[-2000:]
+    bodies = _bodies(out.read_text(), "gemm_splitk_bf16_kernel")
+    assert len(bodies) == 2, "four and eight waves"
+    for name, body in bodies.items():
+        store = next(n for n, l in enumerate(body) if "ds_write_b128" in l)
+        wait = next(l for l in reversed(body[:store]) if "s_waitcnt vmcnt" in l)
+        assert int(re.search(r"vmcnt\((\d+)\)", wait).group(1)) >= 16, f"{name}: {wait.strip()}"
