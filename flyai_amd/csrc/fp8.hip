@@ -373,9 +373,11 @@ int launch_moe_fp8(const uint8_t* aq, const uint8_t* as, const int32_t* perm, co
 }
 
 // ---- combine: out[t] = bf16(residual + bf16(sum_s y[inv[t*k+s]] + shared[t])) ------------------------
-// A thread takes four features of one token; the k rows' loads go out together (a slot past k reads the last one
-// and is not added).  It moves bytes only: with one workgroup a token and one load after the other, 155 tokens of
-// 7,168 x 8 took 26 us, now 6.3.
+// A thread takes four features of one token; the k <= NS rows' loads go out together (a slot past k reads the last
+// one and is not added).  It moves bytes only: with one workgroup a token and one load after the other, 155 tokens of
+// 7,168 x 8 took 26 us, now 6.3.  Eight slots for any k cost the small ones: 4,096 tokens x 7,168 with k = 1 38.9 us
+// and with k = 2 60.6; with as many slots as k 33.7 and 43.2.
+template <int NS>
 __global__ __launch_bounds__(256) void moe_combine_sum_kernel(const uint16_t* __restrict__ y,
                                                               const int32_t* __restrict__ inv, int k,
                                                               int H, const uint16_t* __restrict__ shared,
@@ -383,9 +385,9 @@ __global__ __launch_bounds__(256) void moe_combine_sum_kernel(const uint16_t* __
   const int t = blockIdx.x;
   const int i = blockIdx.y * 256 + threadIdx.x;
   if (i >= H / 4) return;
-  uint2 v[8], sv = make_uint2(0, 0), rv = make_uint2(0, 0);
+  uint2 v[NS], sv = make_uint2(0, 0), rv = make_uint2(0, 0);
 #pragma unroll
-  for (int s = 0; s < 8; ++s) v[s] = reinterpret_cast<const uint2*>(y + (size_t)inv[t * k + min(s, k - 1)] * H)[i];
+  for (int s = 0; s < NS; ++s) v[s] = reinterpret_cast<const uint2*>(y + (size_t)inv[t * k + min(s, k - 1)] * H)[i];
   if (shared) sv = reinterpret_cast<const uint2*>(shared + (size_t)t * H)[i];
   if (residual) rv = reinterpret_cast<const uint2*>(residual + (size_t)t * H)[i];
   float acc[4] = {0.f, 0.f, 0.f, 0.f};
@@ -394,7 +396,7 @@ __global__ __launch_bounds__(256) void moe_combine_sum_kernel(const uint16_t* __
     acc[2] += bf2f(u.y & 0xffff); acc[3] += bf2f(u.y >> 16);
   };
 #pragma unroll
-  for (int s = 0; s < 8; ++s)
+  for (int s = 0; s < NS; ++s)
     if (s < k) add(v[s]);
   if (shared) add(sv);
   if (residual) {
@@ -467,7 +469,13 @@ extern "C" int flyai_moe_combine_sum(const uint16_t* y_perm, const int32_t* inv,
   FLYAI_REQUIRE(T >= 0 && k >= 1 && k <= 8 && H > 0 && H % 4 == 0, "combine_sum: bad shape");
   FLYAI_REQUIRE(y_perm && inv && out, "combine_sum: null pointer");
   if (T == 0) return FLYAI_OK;
-  hipLaunchKernelGGL(moe_combine_sum_kernel, dim3(T, ceil_div(H / 4, 256)), dim3(256), 0, as_stream(stream), y_perm, inv, k, H,
-                     shared, residual, out);
+  auto go = [&](auto ns) {
+    hipLaunchKernelGGL(moe_combine_sum_kernel<decltype(ns)::value>, dim3(T, ceil_div(H / 4, 256)), dim3(256), 0,
+                       as_stream(stream), y_perm, inv, k, H, shared, residual, out);
+  };
+  if (k == 1) go(std::integral_constant<int, 1>{});
+  else if (k == 2) go(std::integral_constant<int, 2>{});
+  else if (k <= 4) go(std::integral_constant<int, 4>{});
+  else go(std::integral_constant<int, 8>{});
   return check_launch("moe_combine_sum");
 }

@@ -234,3 +234,32 @@ def test_deepseek_moe_layer_vs_oracle():
     # the MoE increment alone (the residual dominates the sum)
     mar, cos = _metrics((h.float() - h0.float()).cpu().numpy(), (ref - h0.float().cpu()).numpy())
     assert cos >= COS, f"moe delta cos {cos:.6f}"
+
+
+# ---- combine --------------------------------------------------------------------------------------
+
+@pytest.mark.parametrize("k", [1, 2, 3, 4, 5, 6, 8])
+@pytest.mark.parametrize("T,H,shared,residual", [(3, 4, False, False), (5, 1028, True, False), (2, 1024, False, True),
+                                                 (4, 7168, True, True)])
+def test_combine_sum_bit_exact(k, T, H, shared, residual):
+    """The k rows summed in slot order in fp32, the shared row after them, rounded to bf16, then the residual: bit
+    for bit, with a last block of features that is not whole, every number of slots, and an infinity and a NaN in
+    the last slot's rows (a slot past k is loaded and must not be added)."""
+    from flyai_amd import ops
+    y = torch.randn(T * k, H, device=DEV, generator=_gen(41)).to(torch.bfloat16)
+    inv = torch.randperm(T * k, generator=torch.Generator().manual_seed(k)).to(torch.int32).to(DEV)
+    y[inv[k - 1].long(), 0], y[inv[2 * k - 1].long(), H - 1] = float("inf"), float("nan")
+    sh = torch.randn(T, H, device=DEV, generator=_gen(42)).to(torch.bfloat16) if shared else None
+    res = torch.randn(T, H, device=DEV, generator=_gen(43)).to(torch.bfloat16) if residual else None
+    acc = torch.zeros(T, H, device=DEV)
+    for s in range(k):
+        acc = acc + y[inv.view(T, k)[:, s].long()].float()
+    if shared:
+        acc = acc + sh.float()
+    ref = (res.float() + acc.to(torch.bfloat16).float() if residual else acc).to(torch.bfloat16)
+    got = ops.moe_combine_sum(y, inv, k, shared=sh, residual=res)
+    assert torch.equal(got.isnan(), ref.isnan())
+    ok = ~ref.isnan()
+    assert torch.equal(got[ok].view(torch.int16), ref[ok].view(torch.int16))
+    if residual:  # in place
+        assert torch.equal(ops.moe_combine_sum(y, inv, k, shared=sh, residual=res, out=res).view(torch.int16), got.view(torch.int16))
