@@ -176,6 +176,16 @@ def test_permute_blocks_bit_exact(P, E):
         assert np.array_equal(g.cpu().numpy(), r)
 
 
+@pytest.mark.parametrize("P,first", [(1024, 1024), (2048, 1024), (3000, 1), (5000, 0), (5000, 4999)])
+def test_permute_counts_before_and_after_a_block_bit_exact(P, first):
+    """Long runs of one expert: a block's counts of the ids before it and of the rest are kept apart and added."""
+    from flyai_amd import ops
+    ids = np.where(np.arange(P) < first, 200, 7).astype(np.int32)[:, None]
+    got = ops.moe_permute(torch.tensor(ids, device=DEV), 256)
+    for g, r in zip(got, oroute.permute(ids, 256)):
+        assert np.array_equal(g.cpu().numpy(), r)
+
+
 # the last batch of the one-workgroup kernel and the first of the two launches, per E and selection kernel
 @pytest.mark.parametrize("T,E,k", [(62, 128, 4), (63, 128, 4), (31, 256, 8), (32, 256, 8), (64, 4, 2), (65, 4, 4),
                                    (64, 120, 4), (70, 120, 8), (64, 16, 8), (300, 112, 2)])
