@@ -384,6 +384,18 @@ __global__ __launch_bounds__(256) void grouped_topk_kernel(const float* __restri
   }
 }
 
+// Wide rows (H > 3072): one expert a wave, or two that share the unpacked activations in half as many workgroups of
+// up to twice the length.  Two where that takes fewer rounds over the chip: a CU holds three workgroups of the
+// one-expert kernel (158 registers) and two of the other (215), fewer where their 4 H activations fill its LDS.
+// Logits and selection, one / two: 256 experts x 7,168, 33 tokens (2 rounds / 1) 22.1 / 18.9 us, 155 tokens (5 / 3)
+// 40.5 / 32.7; x 4,096, 48 tokens (1 / 1) 16.1 / 16.3, 64 (2 / 1) 18.6 / 16.3, 68 (2 / 2) 19.4 / 20.7, 128 (3 / 2)
+// 23.8 / 21.7; 128 experts x 4,096, 155 tokens (2 / 2) 19.5 / 20.7.
+inline bool two_experts_a_wave(int T, int H, int E) {
+  const int lds = (int)(160 * 1024 / (4 * H * sizeof(uint16_t))), cus = device_cus();
+  const int one = ceil_div(ceil_div(T, 4) * ceil_div(E, 4), std::min(lds, 3) * cus);
+  return ceil_div(ceil_div(T, 4) * ceil_div(E, 8), std::min(lds, 2) * cus) < one;
+}
+
 int launch_router_grouped(const uint16_t* x, const uint16_t* w, const float* e_bias, int T, int H, int E,
                           int n_group, int topk_group, int k, float route_scale, float* logits,
                           int32_t* ids, float* wts, hipStream_t s) {
@@ -391,12 +403,10 @@ int launch_router_grouped(const uint16_t* x, const uint16_t* w, const float* e_b
   if (H <= 3072)
     hipLaunchKernelGGL((router_logits_kernel<8, 2, 6, false>), dim3(ceil_div(T, 8), ceil_div(E, 8)),
                        dim3(256), 8 * H * sizeof(uint16_t), s, x, w, nullptr, T, H, E, logits);
-  else if (ceil_div(T, 4) * ceil_div(E, 4) > 512)
-    // more workgroups than the chip holds at once (two a CU): two experts a wave share the unpacked activations,
-    // 155 tokens x 256 experts x 7,168 in 31 us where one expert a wave takes 40 (four: 39, one wave a SIMD)
+  else if (two_experts_a_wave(T, H, E))
     hipLaunchKernelGGL((router_logits_kernel<4, 2, 14, false>), dim3(ceil_div(T, 4), ceil_div(E, 8)),
                        dim3(256), 4 * H * sizeof(uint16_t), s, x, w, nullptr, T, H, E, logits);
-  else  // fewer: twice the workgroups, each half as long
+  else
     hipLaunchKernelGGL((router_logits_kernel<4, 1, 14, false>), dim3(ceil_div(T, 4), ceil_div(E, 4)),
                        dim3(256), 4 * H * sizeof(uint16_t), s, x, w, nullptr, T, H, E, logits);
   int rc = check_launch("router_logits(fp32)");

@@ -105,6 +105,14 @@ def test_grouped_router_wide_rows_bit_exact(T, H, E, k):
     assert np.array_equal(ids.cpu().numpy(), rids) and np.array_equal(wts.cpu().numpy(), rwts)
 
 
+@pytest.mark.parametrize("T,H,E,k", [(62, 3592, 252, 6), (64, 4096, 256, 8), (68, 4096, 256, 8), (49, 3080, 256, 4),
+                                     (48, 3080, 256, 4)])
+def test_grouped_router_rounds_rule_bit_exact(T, H, E, k):
+    """The rule counts rounds of workgroups over the chip (by registers and by the LDS of H activations): batches just
+    inside and just past a round of either kernel, a last token group and a last expert pair that are not whole."""
+    test_grouped_router_wide_rows_bit_exact(T, H, E, k)
+
+
 def test_grouped_router_ties_go_to_lower_ids():
     """Zero router weights make every score sigmoid(0) = 0.5; a bias with repeated values then
     leaves ties in both the group scores and the expert choices."""
