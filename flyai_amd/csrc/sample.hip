@@ -150,8 +150,9 @@ __device__ uint32_t radix_select(int V, KeyOf key_of, MassOf mass_of, uint64_t l
 }
 
 // One row by one kSampThreads workgroup, for any logits (NaN, infinities, denormal quotients) and with no
-// workspace: every pass reads the row again.
-__device__ void sample_row_general(SampShared& sh, int row, const uint16_t* __restrict__ logits, int V, float temp,
+// workspace: every pass reads the row again.  Inlined into sample_rows_kernel: a function call there takes 128
+// registers and scratch memory instead of 66 and none (512 greedy rows of 512 logits 32 us instead of 4.9).
+__device__ __forceinline__ void sample_row_general(SampShared& sh, int row, const uint16_t* __restrict__ logits, int V, float temp,
                                    int top_k, float top_p, const int32_t* __restrict__ draft,
                                    const double* __restrict__ u, float* __restrict__ p_draft,
                                    int32_t* __restrict__ draw, float* __restrict__ probs) {
@@ -348,6 +349,16 @@ __global__ __launch_bounds__(kSampThreads) void sample_rows_kernel(
     int32_t* __restrict__ draw, float* __restrict__ probs) {
   __shared__ SampShared sh;
   sample_row_general(sh, blockIdx.x, logits, V, temp, top_k, top_p, draft, u, p_draft, draw, probs);
+}
+
+// The same, called: for the rows that the split path leaves to it, so that its code does not sit among that path's
+// (inlined there one row of 128,256 logits without top-k and top-p takes 19.1 us instead of 18.2).
+__device__ __attribute__((noinline)) void sample_row_general_call(SampShared& sh, int row, const uint16_t* __restrict__ logits,
+                                                                  int V, float temp, int top_k, float top_p,
+                                                                  const int32_t* __restrict__ draft,
+                                                                  const double* __restrict__ u, float* __restrict__ p_draft,
+                                                                  int32_t* __restrict__ draw, float* __restrict__ probs) {
+  sample_row_general(sh, row, logits, V, temp, top_k, top_p, draft, u, p_draft, draw, probs);
 }
 
 // ---- a row split over many workgroups ---------------------------------------------------------------
@@ -731,7 +742,7 @@ __global__ __launch_bounds__(kSampThreads) void sample_final_kernel(
   }
   if (mx.general) {
     __syncthreads();  // every thread has read the union's other side
-    sample_row_general(un.gen, row, logits, p.V, temp, top_k, p.top_p, draft, u, p_draft, draw, probs);
+    sample_row_general_call(un.gen, row, logits, p.V, temp, top_k, p.top_p, draft, u, p_draft, draw, probs);
     return;
   }
   // the boundary key: the first, from the bin's largest down, whose running total exceeds the limit

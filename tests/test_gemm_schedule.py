@@ -151,3 +151,17 @@ def test_projection_activations_do_not_wait_for_the_weights(tmp_path):
         store = next(n for n, l in enumerate(body) if "ds_write_b128" in l)
         wait = next(l for l in reversed(body[:store]) if "s_waitcnt vmcnt" in l)
         assert int(re.search(r"vmcnt\((\d+)\)", wait).group(1)) >= 16, f"{name}: {wait.strip()}"
+
+
+def test_one_workgroup_sampler_calls_no_function(tmp_path):
+    """sample_rows_kernel has the row's code inlined: a call would take the registers and scratch memory of any callee
+    for each of its workgroups."""
+    out = tmp_path / "sample.s"
+    flags = [f for f in B.FLAGS if f != "-fPIC"]
+    r = subprocess.run([HIPCC, *flags, "-S", "--cuda-device-only", "-x", "hip", os.path.join(B.CSRC, "sample.hip"), "-o", str(out)],
+                       capture_output=True, text=True)
+    assert r.returncode == 0, r.stderr[-2000:]
+    text = out.read_text()
+    (body,) = _bodies(text, "sample_rows_kernel").values()
+    assert not [l for l in body if "s_swappc" in l or "scratch_" in l]
+    assert re.search(r"\.amdhsa_kernel _ZN5flyai\d+sample_rows_kernel\w+\n(?:(?!\.end_amdhsa_kernel).*\n)*?\s*\.amdhsa_private_segment_fixed_size 0\n", text)
