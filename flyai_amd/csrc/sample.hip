@@ -387,6 +387,11 @@ constexpr int kChunkStep = kChunkThreads * 8;  // ids of one iteration of a chun
 constexpr int kMinChunk = 2 * kChunkStep;      // two iterations: less, and the launch outweighs the loads
 constexpr int kBins = 2048, kBinKeys = 32;     // key >> 5, key & 31
 constexpr int kRowsAtOnce = 256;               // rows of one set of launches; more rows reuse the workspace
+// Greedy rows of few chunks stay with one workgroup: there is little to divide, and the split path's second launch
+// costs more; a workgroup a row takes any number of rows in one launch.  One workgroup / split, us: V 512 1 row
+// 2.8 / 4.9, 512 rows 5.0 / 11.1; V 8,192 4.6 / 6.0 and 10.9 / 15.8; V 12,288 5.5 / 6.0 and 10.8 / 14.4; V 16,384 1 row
+// 7.0 / 6.1, 256 rows 10.0 / 10.5, 512 14.0 / 15.5; V 20,480 1 row 8.2 / 6.0, 512 16.6 / 16.8, 1,024 44.8 / 35.3.
+inline bool greedy_one_workgroup(int R, int V) { return V <= (R >= kRowsAtOnce ? 4 : 3) * kMinChunk; }
 
 struct SampPlan {
   int V, chunk, n_chunks;
@@ -964,6 +969,11 @@ extern "C" int flyai_sample_rows_ws(const uint16_t* logits, int32_t R, int32_t V
   if (R == 0) return FLYAI_OK;
   FLYAI_REQUIRE(workspace && ((uintptr_t)workspace & 7) == 0, "sample_rows: the workspace must be 8-byte aligned");
   hipStream_t s = as_stream(stream);
+  if (!(temp > 0.f) && greedy_one_workgroup(R, V)) {
+    hipLaunchKernelGGL(sample_rows_kernel, dim3(R), dim3(kSampThreads), 0, s, logits, V, temp, top_k, top_p, draft, u, p_draft,
+                       draw, probs);
+    return check_launch("sample_rows");
+  }
   SampPlan p;
   p.V = V;
   const int steps = (int)(((int64_t)V + (int64_t)kMaxChunks * kChunkStep - 1) / ((int64_t)kMaxChunks * kChunkStep));

@@ -354,7 +354,7 @@ int flyai_sample_rows(const uint16_t* logits, int32_t R, int32_t V, float temp, 
                       const int32_t* draft, const double* u, float* p_draft, int32_t* draw, float* probs,
                       flyai_stream_t stream);
 /* flyai_sample_rows with a device workspace (8-byte aligned, flyai_sample_workspace_bytes(R, V) bytes, not
- * initialised): the same results bit for bit, each row split over many workgroups. */
+ * initialised): the same results bit for bit, each row split over many workgroups where that is faster. */
 size_t flyai_sample_workspace_bytes(int32_t R, int32_t V);
 int flyai_sample_rows_ws(const uint16_t* logits, int32_t R, int32_t V, float temp, int32_t top_k, float top_p,
                          const int32_t* draft, const double* u, float* p_draft, int32_t* draw, float* probs,

@@ -228,3 +228,18 @@ def test_split_rows_equal_one_workgroup_rows(R, V, temp, top_k, top_p):
         torch.cuda.synchronize()
         for n in got:
             assert torch.equal(got[n], want[n]), (t, n, (got[n] != want[n]).nonzero()[:4].tolist())
+
+
+@pytest.mark.parametrize("R", [1, 255, 256, 257])
+@pytest.mark.parametrize("V", [1, 12288, 12289, 16384, 16385])
+def test_greedy_rows_on_both_sides_of_the_split(R, V):
+    """Greedy rows of few ids are one workgroup each, longer ones are split; 256 rows move the line."""
+    from flyai_amd import ops
+    x = _logits(R, V, seed=V + R, ties=True)
+    want = x.float().numpy().argmax(-1)
+    d = torch.from_numpy(np.where(np.arange(R) % 2 == 0, want, V - 1).astype(np.int32))
+    out = ops.sample_rows(x.to(DEV), 0.0, draft=d.to(DEV), want_p_draft=True, want_draw=True, want_probs=True)
+    assert np.array_equal(out["draw"].cpu().numpy(), want)
+    assert np.array_equal(out["p_draft"].cpu().numpy(), (d.numpy() == want).astype(np.float32))
+    p = out["probs"].cpu().numpy()
+    assert (p[np.arange(R), want] == 1).all() and (p.sum(-1) == 1).all()
