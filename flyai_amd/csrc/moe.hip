@@ -1217,14 +1217,21 @@ constexpr int kDenseFrom = 8;
 
 inline bool use_dense(int rows_total, int E) { return (int64_t)rows_total >= (int64_t)kDenseFrom * E; }
 
-// Batches of kMidFrom to kMidTo rows per expert on average take the medium-group kernel alone.  gate_up + down,
-// 128 experts: at 4.7 rows the row-pass kernel takes 302 us and this one 328, at 6.3 348 and 331, at 8 409
-// and 346; at 16 the row-pass and GEMM launches together take 440 and this one 375, at 18 416 and 387; at
-// 22 the GEMM takes 434, and this one would run a second pass for most groups.
-constexpr int kMidFrom = 6, kMidTo = 18;
+// Batches of kMidFrom to kMidTo rows per expert on average take the medium-group kernel alone.  gate_up + down, us,
+// 128 experts, H = I = 2880, even routing, without / with it: 5 rows 293 / 306, 6 rows 318 / 302, 8 374 / 312, 12 386 / 330,
+// 18 382 / 357, 19 384 / 360, 20 389 / 414, 22 395 / 426: from 20 rows on a group or two pass 32 rows, and a second pass's units
+// start another round of workgroups.  With half of the rows on a tenth of the experts: 6 rows 424 / 365, 8 368 / 373,
+// 10.4 358 / 386, 12 362 / 390, 14 414 / 405, 18 469 / 423: from 8 to 13 rows it loses 1 to 8 % there (the other groups have
+// 4 to 8 rows, the row pass's best) and wins 17 to 21 % on even batches, and the host sees only the average.  Leaving
+// groups over 32 rows to the 96-row GEMM costs even batches 3 % and skewed ones of 32 experts 30 %.
+// Where the kernel's units of one block fill less than half of the CUs it starts at kMidFewFrom: 4 experts of 6 rows 28.6
+// without, 35.1 with it, 12 rows 43.8 / 35.2; 8 experts' down of 6 rows 13.7 / 17.7, of 8 32.6 / 17.7.
+constexpr int kMidFrom = 6, kMidFewFrom = 8, kMidTo = 18;
 
-inline bool use_mid(int rows_total, int E, int K) {
-  return K >= 128 && K <= 4064 && (int64_t)rows_total >= (int64_t)kMidFrom * E && (int64_t)rows_total < (int64_t)kMidTo * E;
+inline bool use_mid(int rows_total, int E, int N, int K) {
+  const int64_t units = (int64_t)E * ceil_div(mx_geom(E, N, K).NT, kGemmTiles);
+  const int from = 2 * units >= device_cus() ? kMidFrom : kMidFewFrom;
+  return K >= 128 && K <= 4064 && (int64_t)rows_total >= (int64_t)from * E && (int64_t)rows_total < (int64_t)kMidTo * E;
 }
 
 // whether a batch of rows_total permuted rows gives any expert group to the dense kernels
@@ -1237,7 +1244,7 @@ int launch_moe_gate_up(const uint16_t* x, const int32_t* perm, const int32_t* of
                        const uint8_t* w13, const float* b13, int T, int E, int H, int I, uint16_t* h,
                        hipStream_t s) {
   const MxGeom gm = mx_geom(E, 2 * I, H);
-  if (use_mid(T * k_top, E, H)) return launch_moe_mid<true>(x, perm, offsets, k_top, w13, b13, T * k_top, E, 2 * I, H, h, s);
+  if (use_mid(T * k_top, E, 2 * I, H)) return launch_moe_mid<true>(x, perm, offsets, k_top, w13, b13, T * k_top, E, 2 * I, H, h, s);
   const bool dense = use_dense(T * k_top, E) && H >= 128;  // the tiled kernel reads 128-K groups
   if (H <= 4064) {
     const int wg_per_e = ceil_div(gm.NT, 4 * kNTWGateUp);
@@ -1260,7 +1267,7 @@ int launch_moe_gate_up(const uint16_t* x, const int32_t* perm, const int32_t* of
 int launch_moe_down(const uint16_t* h, const int32_t* offsets, const uint8_t* w2, const float* b2,
                     int rows_total, int E, int H, int I, float* y, hipStream_t s) {
   const MxGeom gm = mx_geom(E, H, I);
-  if (use_mid(rows_total, E, I)) return launch_moe_mid<false>(h, nullptr, offsets, 1, w2, b2, rows_total, E, H, I, y, s);
+  if (use_mid(rows_total, E, H, I)) return launch_moe_mid<false>(h, nullptr, offsets, 1, w2, b2, rows_total, E, H, I, y, s);
   const bool dense = use_dense(rows_total, E) && I >= 128;  // the tiled kernel reads 128-K groups
   if (I <= 4064) {
     const int wg_per_e = ceil_div(gm.NT, 4 * kNTWDown);

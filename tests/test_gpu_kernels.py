@@ -869,6 +869,39 @@ def test_medium_group_experts_bit_identical(H, I):
         assert torch.equal(h.view(torch.int16), h_all[rows].view(torch.int16)), "gate_up differs"
         assert torch.equal(y.view(torch.int32), y_all[rows].view(torch.int32)), "down differs"
 
+def _expert_batches_equal_parts(ids, H, I, E, part, seed):
+    """gate_up and down of a batch of `ids` [T, k] against the same tokens in batches of `part`, bit for bit."""
+    from flyai_amd import ops
+    from flyai_amd.weights import GptOssShape, synthetic_moe
+    m = synthetic_moe(GptOssShape(hidden=H, intermediate=I, n_experts=E), _gen(seed), DEV)
+    w13 = ops.mxfp4_repack(m["w13_blocks"], m["w13_scales"])
+    w2 = ops.mxfp4_repack(m["w2_blocks"], m["w2_scales"])
+    T, k = ids.shape
+    x = _rms_input(T, H, seed + 1)
+    x[T // 2, 1], x[T - 1, H - 1] = float("inf"), float("nan")
+
+    def run(rows):
+        _, off, perm, inv = ops.moe_permute(ids[rows].contiguous(), E)
+        h = ops.moe_gate_up(x[rows].contiguous(), perm, off, k, w13, m["b13"], E, I)
+        return (h[inv.long()].view(len(rows), k, I).view(torch.int16),
+                ops.moe_down(h, off, w2, m["b2"], E, H)[inv.long()].view(len(rows), k, H).view(torch.int32))
+
+    h_all, y_all = run(torch.arange(T, device=DEV))
+    for t0 in range(0, T, part):
+        rows = torch.arange(t0, min(T, t0 + part), device=DEV)
+        h, y = run(rows)
+        assert torch.equal(h, h_all[rows]), "gate_up differs"
+        assert torch.equal(y, y_all[rows]), "down differs"
+
+
+@pytest.mark.parametrize("sizes", [(6, 6, 6, 6), (7, 9, 8, 7), (8, 8, 9, 8), (1, 17, 0, 6, 33, 8, 2, 1)])
+def test_few_experts_medium_rule_bit_identical(sizes):
+    """Where the medium-group kernel's units leave most of the chip idle it starts at 8 rows per expert: batches on
+    both sides of that line and on it, against batches of the row-pass kernel."""
+    T = sum(sizes)
+    ids = torch.cat([torch.full((n,), e) for e, n in enumerate(sizes)])[torch.randperm(T, generator=torch.Generator().manual_seed(5))]
+    _expert_batches_equal_parts(ids.to(torch.int32).to(DEV)[:, None], 544, 1024, len(sizes), 5 * len(sizes), 71)
+
 
 @pytest.mark.parametrize("H", [32, 128, 160, 288, 2880])
 @pytest.mark.parametrize("n,V", [(1, 16), (16, 144), (17, 272), (48, 128), (64, 1040)])
