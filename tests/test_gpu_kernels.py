@@ -869,6 +869,24 @@ def test_medium_group_experts_bit_identical(H, I):
         assert torch.equal(h.view(torch.int16), h_all[rows].view(torch.int16)), "gate_up differs"
         assert torch.equal(y.view(torch.int32), y_all[rows].view(torch.int32)), "down differs"
 
+@pytest.mark.parametrize("K", [32, 160, 2880])
+def test_mxfp4_repack_leaves_padding_scales_zero(K):
+    """The tiled expert kernels multiply the padding of K with zero activations and rely on its scale bytes for finite
+    weights: the re-pack writes zeros there, whatever the real scales are and whatever the buffer held."""
+    from flyai_amd import ops
+    E, N, G = 2, 48, K // 32
+    blocks = torch.full((E, N, G, 16), 0xff, dtype=torch.uint8, device=DEV)
+    del_me = torch.full((ops.mxfp4_packed_bytes(E, N, K),), 0xff, dtype=torch.uint8, device=DEV)
+    del del_me  # the allocator hands the re-pack this memory
+    packed = ops.mxfp4_repack(blocks, torch.full((E, N, G), 0xff, dtype=torch.uint8, device=DEV)).cpu().numpy()
+    KG4 = (G + 15) // 16  # scale words of 4 groups of 4 blocks
+    words = packed[E * N * G * 16:].reshape(E * N // 16, KG4, 4, 16, 4)  # [tile][word][block of a group][row][group]
+    for kg in range(4 * KG4):
+        for g in range(4):
+            want = 0xff if 4 * kg + g < G else 0
+            assert (words[:, kg // 4, g, :, kg % 4] == want).all(), (kg, g)
+
+
 def _expert_batches_equal_parts(ids, H, I, E, part, seed):
     """gate_up and down of a batch of `ids` [T, k] against the same tokens in batches of `part`, bit for bit."""
     from flyai_amd import ops
