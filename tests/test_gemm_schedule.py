@@ -90,35 +90,44 @@ def test_group_loops_issue_exact_groups(gemm_asm):
         assert seen == Counter({1: 1, 2: 2, 3: 2})
 
 
+def _check_prologues(name, body, expected):
+    checked = 0
+    for w, line in enumerate(body):
+        m = re.search(r"s_waitcnt vmcnt\((15|18|21)\)", line)
+        if not m:
+            continue
+        loads = int(m.group(1)) // 3
+        md = loads - 4
+        ops = []
+        for n in range(w - 1, -1, -1):
+            t = body[n].strip()
+            if t.startswith("s_waitcnt vmcnt(0)") or t.startswith("s_barrier"):
+                break
+            mm = VMEM.match(body[n])
+            if mm:
+                ops.append(mm.group(1))
+        ops.reverse()
+        # the youngest 3 groups must be whole groups; if fewer loads follow the last drain, the
+        # loads before it are complete and the rest must be the tail of one group
+        whole = min(3, len(ops) // loads)
+        for g in range(whole):
+            chunk = ops[len(ops) - (g + 1) * loads:len(ops) - g * loads]
+            assert Counter(chunk) == _group(md), f"{name} MD={md}: {ops}"
+        if whole < 3:
+            head = Counter(ops[:len(ops) - whole * loads])
+            assert not head - _group(md), f"{name} MD={md}: {ops}"
+        checked += 1
+    assert checked == expected, f"{name}: expected one prologue wait per row-tile count"
+
+
 def test_prologue_issues_groups_in_order(gemm_asm):
     for name, body in gemm_asm.items():
-        checked = 0
-        for w, line in enumerate(body):
-            m = re.search(r"s_waitcnt vmcnt\((15|18|21)\)", line)
-            if not m:
-                continue
-            loads = int(m.group(1)) // 3
-            md = loads - 4
-            ops = []
-            for n in range(w - 1, -1, -1):
-                t = body[n].strip()
-                if t.startswith("s_waitcnt vmcnt(0)") or t.startswith("s_barrier"):
-                    break
-                mm = VMEM.match(body[n])
-                if mm:
-                    ops.append(mm.group(1))
-            ops.reverse()
-            # the youngest 3 groups must be whole groups; if fewer loads follow the last drain, the
-            # loads before it are complete and the rest must be the tail of one group
-            whole = min(3, len(ops) // loads)
-            for g in range(whole):
-                chunk = ops[len(ops) - (g + 1) * loads:len(ops) - g * loads]
-                assert Counter(chunk) == _group(md), f"{name} MD={md}: {ops}"
-            if whole < 3:
-                head = Counter(ops[:len(ops) - whole * loads])
-                assert not head - _group(md), f"{name} MD={md}: {ops}"
-            checked += 1
-        assert checked == 5, f"{name}: expected one prologue wait per row-tile count"
+        _check_prologues(name, body, 5)
+
+
+def test_medium_prologue_issues_groups_in_order(gemm_asm_mid):
+    for name, body in gemm_asm_mid.items():
+        _check_prologues(name, body, 2)
 
 
 def test_medium_kernel_groups(gemm_asm_mid):

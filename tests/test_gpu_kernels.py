@@ -843,7 +843,7 @@ def test_medium_group_experts_bit_identical(H, I):
     """A batch of 6 to 18 rows per expert on average runs the medium-group kernel; the same rows in batches
     of at most 5 per expert run the row-pass kernel: h and y equal bit for bit.  Groups of 0 rows, of one
     row tile and its neighbours, of two and their neighbours, and of more than a pass; K of whole and partial
-    128-K groups; fewer weight blocks than a chunk; rows holding an infinity (first and last group) and a NaN."""
+    128-K groups; one weight block a unit; rows holding an infinity (first and last group) and a NaN."""
     from flyai_amd import ops
     from flyai_amd.weights import GptOssShape, synthetic_moe
     sizes = [1, 15, 0, 16, 17, 32, 33, 14]
@@ -910,6 +910,22 @@ def _expert_batches_equal_parts(ids, H, I, E, part, seed):
         h, y = run(rows)
         assert torch.equal(h, h_all[rows]), "gate_up differs"
         assert torch.equal(y, y_all[rows]), "down differs"
+
+
+@pytest.mark.parametrize("skewed", [False, True])
+def test_medium_group_experts_full_size_bit_identical(skewed):
+    """The medium-group kernel with three weight blocks a unit (128 experts, H = I = 2880: a chunk's later blocks, the
+    ring running over them, their bias, a last chunk of two blocks): 333 tokens against batches of the row-pass
+    kernel, with even routing and with half of the rows on a tenth of the experts (groups of two and more passes)."""
+    E, k, T = 128, 4, 333
+    g = torch.Generator().manual_seed(7)
+    p = torch.ones(E)
+    if skewed:
+        p[torch.randperm(E, generator=g)[:E // 10]] = 9.0
+    ids = (-torch.rand(T, E, generator=g).log() / p).topk(k, 1, largest=False)[1].sort(1)[0].to(torch.int32)
+    most = int(torch.bincount(ids.flatten(), minlength=E).max())
+    assert 6 * E <= T * k < 18 * E and (most > 32) == skewed
+    _expert_batches_equal_parts(ids.to(DEV), 2880, 2880, E, 150, 73)
 
 
 @pytest.mark.parametrize("sizes", [(6, 6, 6, 6), (7, 9, 8, 7), (8, 8, 9, 8), (1, 17, 0, 6, 33, 8, 2, 1)])

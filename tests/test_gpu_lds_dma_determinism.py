@@ -1,8 +1,9 @@
 """The kernels that fill LDS with direct-to-LDS loads (global_load_lds) repeat bit for bit.
 
-Three kernels stage operands global -> LDS directly and read a stage once an explicit ``vmcnt`` wait
+Four kernels stage operands global -> LDS directly and read a stage once an explicit ``vmcnt`` wait
 says its loads have landed: the dense MXFP4 expert GEMM (``moe_mxfp4_gemm_kernel``), its scaled-MFMA
-twin (``moe_mx_gemm_kernel``) and the prefill-sized projection GEMM (``gemm_tiled_lds_kernel``).  A
+twin (``moe_mx_gemm_kernel``), the medium-group expert kernel (``moe_mxfp4_mid_kernel``, at 333 rows) and the
+prefill-sized projection GEMM (``gemm_tiled_lds_kernel``).  A
 stage read before its loads had written LDS would show up as a few wrong 16 x 16 output tiles now and
 then, not every time.  Each kernel therefore runs many times on fixed inputs at the prefill-chunk
 shape (2096 rows; 128 experts at about 65 rows each), and every output must equal the first bit for
@@ -74,6 +75,18 @@ def test_scaled_mfma_expert_gemm_repeats_bit_identical(c2_experts):
     hq, hs = ops.mx_act_quant(h)
     _repeat_identical(lambda: ops.moe_down_fp8act(h, hq, hs, off, w2, m["b2"], E, H), REPS // 2,
                       "moe_mx_gemm_kernel (down)")
+
+
+def test_medium_expert_kernel_repeats_bit_identical(c2_experts):
+    """333 tokens: about ten rows an expert, three weight blocks a unit."""
+    from flyai_amd import ops
+    shape, m, w13, w2, x, _, _ = c2_experts
+    E, H, I, k = shape.n_experts, shape.hidden, shape.intermediate, shape.top_k
+    x = x[:333].contiguous()
+    ids = torch.rand(333, E, device=DEV, generator=_gen(6)).topk(k, 1)[1].sort(1)[0].to(torch.int32)
+    _, off, perm, _ = ops.moe_permute(ids, E)
+    h = _repeat_identical(lambda: ops.moe_gate_up(x, perm, off, k, w13, m["b13"], E, I), REPS, "moe_mxfp4_mid_kernel (gate_up)")
+    _repeat_identical(lambda: ops.moe_down(h, off, w2, m["b2"], E, H), REPS, "moe_mxfp4_mid_kernel (down)")
 
 
 @pytest.mark.parametrize("N,K", [(5120, 2880), (2880, 4096)])
