@@ -328,66 +328,4 @@ __device__ __forceinline__ void topk_softmax_lane(const float* __restrict__ lrow
   }
 }
 
-// The same top-k + softmax by a whole wave (E <= 256): each lane holds E/64 logits; K rounds of a
-// wave-wide argmax over (value desc, id asc) give the same selection in the same order as
-// topk_softmax_lane, and every lane then does the identical softmax / id sort, so ids and weights
-// are bit-identical to it.  Lanes 0..K-1 write the outputs.
-template <int K>
-__device__ __forceinline__ void topk_softmax_wave_vals(const float (&v)[4], int E, int lane,
-                                                       int32_t* ids_out, float* w_out) {
-  bool taken[4];
-#pragma unroll
-  for (int j = 0; j < 4; ++j) taken[j] = 4 * lane + j >= E;
-  float sv[K];
-  int si[K];
-#pragma unroll
-  for (int r = 0; r < K; ++r) {
-    float bv = -INFINITY;
-    int bi = 0x7fffffff;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int e = 4 * lane + j;
-      if (!taken[j] && (v[j] > bv || (v[j] == bv && e < bi))) { bv = v[j]; bi = e; }
-    }
-#pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) {
-      const float ov = __shfl_xor(bv, o, 64);
-      const int oi = __shfl_xor(bi, o, 64);
-      if (ov > bv || (ov == bv && oi < bi)) { bv = ov; bi = oi; }
-    }
-    sv[r] = bv;
-    si[r] = bi;
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-      if (4 * lane + j == bi) taken[j] = true;
-  }
-  float ex[K], sum = 0.f;
-#pragma unroll
-  for (int j = 0; j < K; ++j) { ex[j] = expf(sv[j] - sv[0]); sum += ex[j]; }
-  sort_ids_with_weights<K>(si, ex);
-#pragma unroll
-  for (int j = 0; j < K; ++j)
-    if (lane == j) {
-      ids_out[j] = (unsigned)si[j] < (unsigned)E ? si[j] : 0;  // a NaN row selects nothing: expert 0
-      w_out[j] = ex[j] / sum;
-    }
-}
-
-// lane l's logits of a row: experts 4l .. 4l+3 (-inf past E)
-__device__ __forceinline__ void load_logits_lane(const float* __restrict__ lrow, int E, int lane, float (&v)[4]) {
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const int e = 4 * lane + j;
-    v[j] = e < E ? lrow[e] : -INFINITY;
-  }
-}
-
-template <int K>
-__device__ __forceinline__ void topk_softmax_wave(const float* __restrict__ lrow, int E, int lane,
-                                                  int32_t* ids_out, float* w_out) {
-  float v[4];
-  load_logits_lane(lrow, E, lane, v);
-  topk_softmax_wave_vals<K>(v, E, lane, ids_out, w_out);
-}
-
 }  // namespace flyai

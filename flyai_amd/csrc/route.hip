@@ -621,8 +621,6 @@ __global__ __launch_bounds__(kPermBlock) void moe_topk_permute_kernel(
 int launch_permute(const int32_t* ids, int T, int k, int E, int32_t* hist, int32_t* offsets,
                    int32_t* perm, int32_t* inv, hipStream_t s);
 
-int launch_topk(const float* logits, int T, int E, int k, int32_t* ids, float* wts, hipStream_t s);
-
 // Top-k + softmax of precomputed logits, then histogram / permute: one workgroup for a small batch,
 // else a launch of each over the whole chip.
 int launch_topk_permute(const float* logits, int T, int E, int k, int32_t* ids, float* wts, int32_t* hist,

@@ -80,9 +80,9 @@ int flyai_router_topk_softmax(const uint16_t* x, const uint16_t* w, const uint16
 int flyai_moe_permute(const int32_t* topk_ids, int32_t T, int32_t k, int32_t E, int32_t* hist,
                       int32_t* offsets, int32_t* perm, int32_t* inv, flyai_stream_t stream);
 
-/* a2 + a3 in one call (the stage's path): router logits, then -- for a small batch (up to 64
- * tokens) -- top-k of every token and the histogram / permute in a single one-workgroup kernel (one
- * kernel each above that).
+/* a2 + a3 in one call (the stage's path): router logits, then -- for a small batch (T <= 64 and
+ * T*(E+4) <= 8192, what the kernel's LDS holds: 62 tokens of 128 experts, 31 of 256) -- top-k of every
+ * token and the histogram / permute in a single one-workgroup kernel (one kernel each above that).
  * Same outputs and bit-exact indices as flyai_router_topk_softmax followed by flyai_moe_permute. */
 int flyai_moe_route_permute(const uint16_t* x, const uint16_t* w, const uint16_t* b, int32_t T,
                             int32_t H, int32_t E, int32_t k, int32_t* topk_ids, float* topk_w,
