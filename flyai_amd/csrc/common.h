@@ -217,9 +217,9 @@ constexpr uint32_t kBufOutside = 0x80000000u;
 // A wave-uniform value, in a scalar register.  Some uniform integers (a clamp, the wave's number) come from
 // vector instructions, and a buffer resource built from one that stays in a vector register makes the
 // compiler wrap every load through it in a loop over the wave's "different" resources: a dozen
-// instructions a load, and no scheduling across it.  Decode expert kernels with and without those loops
-// (128 experts, top-4, H = I = 2880): 56 tokens 161 -> 147 us gate_up and 86 -> 80 us down, 12 tokens 63.6 ->
-// 59.9 and 39.9 -> 36.8, 200 tokens 243 -> 221 and 134 -> 127.
+// instructions a load, and no scheduling across it.  With this and the launch cut to the groups that have rows
+// (nth_group in moe.hip), the decode expert kernels (128 experts, top-4, H = I = 2880), gate_up / down: 12 tokens
+// 61.9 -> 59.3 and 37.7 -> 30.2 us, 56 tokens 143.4 -> 138.6 and 78.2 -> 75.4.
 __device__ __forceinline__ int scalar(int v) { return __builtin_amdgcn_readfirstlane(v); }
 
 // 16 bytes through a buffer resource, nontemporal

@@ -782,11 +782,11 @@ __global__ __launch_bounds__(512) void moe_mxfp4_gemm_kernel(
 // Between the row-pass kernel, whose weight stream is read once per 8 rows, and the 96-row GEMM, whose one
 // workgroup a CU holds too few loads in flight to stream the weights of groups this small: the GEMM's pass
 // over at most two row tiles (32 rows), whose stages and registers are small enough for two workgroups of
-// 8 waves a CU (57 KB of LDS, 107-114 registers).  It serves every group of the batch, larger ones in
-// passes of 32 rows.  Same MFMA, K-to-lane mapping and order per output element as the other two, so the
-// same bits.  Rows an expert on average, 128 experts, H = I = 2880, before (row-pass and GEMM launches) and
-// with this kernel, gate_up / down: 6.3 rows 221 / 127 -> 213 / 117 us, 10.4 293 / 163 -> 225 / 125,
-// 16 279 / 161 -> 243 / 132.  What bounds it is the weight stream (5.0-5.4 TB/s).
+// 8 waves a CU (54,276 bytes of LDS, 110 registers for gate_up and 116 for down).  It serves every group of the
+// batch, larger ones in passes of 32 rows.  Same MFMA, K-to-lane mapping and order per output element as the other two,
+// so the same bits.  Rows an expert on average, 128 experts, H = I = 2880, even routing, row-pass and GEMM launches before
+// and this kernel, gate_up / down: 6.5 rows 222 / 127 -> 195 / 111 us, 10.4 261 / 151 -> 206 / 117, 16 247 / 144 -> 226 / 123.
+// What bounds it is the weight stream (5.5 and 4.8 TB/s at 10.4 rows).
 constexpr int kMidRows = 32;
 constexpr int kMidChunk = 3;  // weight blocks a unit: 2 to 6 within 3 % for gate_up; down 117 us with 3, 122-136 with 1, 2, 4, 6
 
@@ -1210,9 +1210,11 @@ int launch_moe_mid(const uint16_t* act, const int32_t* perm, const int32_t* offs
   return check_launch(GATE_UP ? "moe_gate_up_mxfp4(mid)" : "moe_down_mxfp4(mid)");
 }
 
-// Groups of more than kDenseFrom rows take the dense kernel when the batch averages at least that
-// many rows per expert (otherwise the row-pass kernel serves every group: a rare large group costs
-// extra passes, not a launch of mostly idle workgroups).  Both kernels are correct for any count.
+// Which kernels a batch takes, by its rows per expert on average.  With bf16 activations and K of 128 to 4,064 (use_mid):
+// below kMidFrom the row-pass kernel alone, up to kMidTo the medium-group kernel alone, from there on the row-pass
+// kernel for groups of up to kDenseFrom rows and the GEMM for larger ones.  With fp8 activations, and with a longer K, the
+// two share a batch from kDenseFrom rows on average (a rare large group below that costs extra passes, not a launch of
+// mostly idle workgroups).  All are correct for any count.
 constexpr int kDenseFrom = 8;
 
 inline bool use_dense(int rows_total, int E) { return (int64_t)rows_total >= (int64_t)kDenseFrom * E; }
