@@ -172,9 +172,11 @@ constexpr float kMaxSlack = 8.f;
 constexpr float kMaxSentinel = -1e29f;  // a running max at or below this is the initial -1e30 (no key yet)
 
 // The scores s of one 64-key block and row (its position, and in a tree its node): keys outside the row's range
-// become -inf; returns the row's largest (all four lane groups hold it).  rows_block has the same steps written out:
-// called from there the one-wave tree kernel takes 336 registers instead of 320, and 28.2 us instead of 26.2 for 18
-// nodes over 8,000 keys; with the row by reference the four-wave one takes 20.4 instead of 19.3 over 3,000.
+// become -inf; returns the row's largest (all four lane groups hold it).  rows_block calls it for decode rows (16
+// single-token rows of up to 32,768 keys 42.7 us, 46.1 with the steps written out there) and has the steps of a tree
+// written out: called from there the one-wave tree kernel takes 336 registers instead of 320, and 28.2 us instead of 26.2
+// for 18 nodes over 8,000 keys.  With the row by reference the four-wave tree kernel takes 20.4 us instead of 19.3 over
+// 3,000.
 template <bool TREE>
 __device__ __forceinline__ float row_mask_max(bool qval, int qpos, int qnode, f32x4_t (&s)[4], int kb, bool interior,
                                               int key_lo, int key_hi, int window, const TreeView& tv) {
@@ -231,7 +233,6 @@ __device__ __forceinline__ void rows_block(QRows<QT>& R, const uint4 (&kc)[4][2]
                                            const TreeView& tv) {
   const int g = (threadIdx.x & 63) >> 4;
   const float scale = 0.125f * kLog2e;
-  const int tstart = TREE ? tv.start : 0;
   const bf16x8_t ones = as_bf16x8(make_uint4(0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u));
   if (kb + 64 > key_hi) {
 #pragma unroll
@@ -247,21 +248,23 @@ __device__ __forceinline__ void rows_block(QRows<QT>& R, const uint4 (&kc)[4][2]
       s[kt] = mfma16x16x32(as_bf16x8(kc[kt][0]), R.qf[qt][0], f32x4_t{0.f, 0.f, 0.f, 0.f});
       s[kt] = mfma16x16x32(as_bf16x8(kc[kt][1]), R.qf[qt][1], s[kt]);
     }
-    // lane holds S^T[key kb + tile_key(kt, 4g + v)][qrow n]
-    float bmax = -INFINITY;
-    if (interior && R.qval[qt]) {
+    float bmax;
+    if constexpr (!TREE) {
+      bmax = row_mask_max<false>(R.qval[qt], R.qpos[qt], 0, s, kb, interior, key_lo, key_hi, window, tv);
+    } else {  // the same steps, written out
+      // lane holds S^T[key kb + tile_key(kt, 4g + v)][qrow n]
+      bmax = -INFINITY;
+      if (interior && R.qval[qt]) {
 #pragma unroll
-      for (int kt = 0; kt < 4; ++kt)
+        for (int kt = 0; kt < 4; ++kt)
 #pragma unroll
-        for (int v = 0; v < 4; ++v) bmax = fmaxf(bmax, s[kt][v]);
-    } else {
-      const int p = R.qpos[qt];
-      const int lo = max(key_lo, window > 0 ? p - window + 1 : 0);
-      const int hi = min(p, key_hi - 1);
-      // tree: bits [kb - start, kb - start + 64) of the row's mask (key kb + t is bit t)
-      uint64_t tbits = 0;
-      if (TREE) {
-        const int j0 = kb - tstart;
+          for (int v = 0; v < 4; ++v) bmax = fmaxf(bmax, s[kt][v]);
+      } else {
+        const int p = R.qpos[qt];
+        const int lo = max(key_lo, window > 0 ? p - window + 1 : 0);
+        // bits [kb - start, kb - start + 64) of the row's mask (key kb + t is bit t)
+        uint64_t tbits = 0;
+        const int j0 = kb - tv.start;
         if (R.qval[qt] && j0 > -64 && j0 < tv.n) {
           const int wq = j0 >> 6, sh = j0 & 63;  // floor division (j0 may be negative)
           const uint64_t* mrow = tv.mask + (size_t)R.qnode[qt] * tv.words;
@@ -269,27 +272,22 @@ __device__ __forceinline__ void rows_block(QRows<QT>& R, const uint4 (&kc)[4][2]
           const uint64_t w1 = wq + 1 < tv.words ? mrow[wq + 1] : 0ull;
           tbits = sh == 0 ? w0 : (w0 >> sh) | (w1 << (64 - sh));
         }
-      }
 #pragma unroll
-      for (int kt = 0; kt < 4; ++kt)
+        for (int kt = 0; kt < 4; ++kt)
 #pragma unroll
-        for (int v = 0; v < 4; ++v) {
-          const int key = kb + tile_key(kt, 4 * g + v);
-          bool ok;
-          if (TREE) {
-            if (key < tstart)
+          for (int v = 0; v < 4; ++v) {
+            const int key = kb + tile_key(kt, 4 * g + v);
+            bool ok;
+            if (key < tv.start)
               ok = key >= lo && key < key_hi;  // committed prefix (window on positions)
             else  // tree slot: the mask (its window already applied for sliding layers)
               ok = key >= key_lo && key < key_hi && ((tbits >> tile_key(kt, 4 * g + v)) & 1ull);
-            ok = ok && R.qval[qt];
-          } else {
-            ok = R.qval[qt] && key >= lo && key <= hi;
+            s[kt][v] = ok && R.qval[qt] ? s[kt][v] : -INFINITY;
+            bmax = fmaxf(bmax, s[kt][v]);
           }
-          s[kt][v] = ok ? s[kt][v] : -INFINITY;
-          bmax = fmaxf(bmax, s[kt][v]);
-        }
+      }
+      bmax = max_lane_groups(bmax);
     }
-    bmax = max_lane_groups(bmax);
     // (a fully masked row keeps m = -1e30: -1e30 + kMaxSlack rounds to -1e30 and -inf never exceeds it)
     const float m_blk = bmax * scale;
     const bool move = m_blk > R.m_run[qt] + kMaxSlack;
