@@ -759,7 +759,7 @@ constexpr int kCoopNB1 = 2, kCoopNB2 = 1;
 //   4 tokens (two row tiles): 2 blocks, 64 items 7.5 / 7.6, 512 items 8.2 / 9.4; 3 blocks, 64 items 8.8 / 7.8; 4
 //   blocks, 512 items 12.1 / 11.0.
 constexpr int kSoloBlocks2 = 2;
-__device__ __forceinline__ int solo_blocks(int ntok, int full) { return ntok > 2 ? kSoloBlocks2 : full ? 5 : ntok == 2 ? 4 : 3; }
+__host__ __device__ __forceinline__ constexpr int solo_blocks(int ntok, int full) { return ntok > 2 ? kSoloBlocks2 : full ? 5 : ntok == 2 ? 4 : 3; }
 
 union CoopAny {
   CoopShared<1, kCoopNB1> one;
@@ -1083,13 +1083,27 @@ __global__ __launch_bounds__(256) void attn_merge_kernel(const float* __restrict
   *reinterpret_cast<uint4*>(o) = make_uint4(wv[0], wv[1], wv[2], wv[3]);
 }
 
-// Four waves take an item while all the launch's workgroups are on the chip at once: two a CU of the decode kernel
-// (249 registers a wave), one of the tree kernel (336).  Past that the workgroups queue behind one another, where
-// one wave an item (8 and 4 items a CU at once) still has its turn.  One wave / four waves an item, items of 16 blocks
-// of one token: 16 items 16.0 / 9.3 us, 128 24.7 / 15.1, 256 25.8 / 17.0, 512 30.3 / 26.1, 640 32.1 / 34.7; of four tokens
-// and 2 blocks, 640 items: 8.6 / 12.3.  Trees over 8,000 keys: 18 nodes (320 items) 25.9 / 32.6 us, 32 nodes (512 items)
-// 28.5 / 36.8; over 3,000 keys 32 nodes (192 items) 33.1 / 20.8.
-inline int coop_items(bool tree) { return (tree ? 1 : 2) * device_cus(); }
+// Whether four waves take an item (attn_coop_kernel, attn_tree_coop_kernel) or one.  Four while all the launch's
+// workgroups are on the chip at once: two a CU of the decode kernel (249 registers a wave), one of the tree kernel (324).
+// Past that the workgroups queue behind one another, where one wave an item (8 and 4 items a CU at once) still has its
+// turn.  One wave / four waves an item, items of 16 blocks of one token: 16 items 16.0 / 9.3 us, 128 24.7 / 15.1, 256 25.8 /
+// 17.0, 512 30.3 / 26.1.  Trees over 8,000 keys: 18 nodes (320 items) 25.9 / 32.6 us, 32 nodes (512 items) 28.5 / 36.8; over
+// 3,000 keys 32 nodes (192 items) 33.1 / 20.8.
+// The items of a full layer are long and of different lengths, so a queue half as long as the chip still fills up:
+// contexts of 128 to 3,000 keys, 560 items of one token 30.4 / 26.6 us, of four 32.5 / 27.9; up to 1,000 keys, 640 items
+// 26.7 / 23.7 and 28.6 / 24.9; equal contexts of 1,024 keys, 640 items of one, two, four tokens 31.9 / 34.2, 34.6 / 32.2,
+// 38.9 / 37.4; of 128 keys and four tokens 8.6 / 12.3; 880 items of 16 blocks 39.8 / 41.1.  A sliding layer's 640 items of
+// four tokens take 12.2 / 14.4.
+// Where every item would be left to one wave (solo_blocks) it is launched so: a window of 128, one token, 16 to 96 items
+// 6.6 / 6.8 us, 128 6.7 / 7.2.
+inline bool four_waves_an_item(int n_items, int n_small, int window, bool tree) {
+  const int cus = device_cus();
+  if (tree) return n_items <= cus;
+  if (window == 0) return 2 * (int64_t)n_items <= 5 * (int64_t)cus;
+  // an item of up to two tokens spans window + 1 keys: at most (window + 63) / 64 + 1 blocks
+  if (n_small == n_items && (window + 63) / 64 + 1 <= solo_blocks(1, 0)) return false;
+  return n_items <= 2 * cus;
+}
 
 // n_items / n_groups size the grids; counts (nullable) holds this step's live item and group
 // counts on the device, for launches sized by a plan capacity (graph replay)
@@ -1099,8 +1113,8 @@ int launch_attn(const uint16_t* q, const uint16_t* k_pool, const uint16_t* v_poo
                 const flyai_attn_group* groups, int n_groups, const int32_t* counts, float* partials,
                 uint16_t* out, const flyai_attn_tree* tree, bool merge, hipStream_t s) {
   if (n_items == 0) return FLYAI_OK;
-  (void)n_small;  // the plan's two ranges share one launch
-  const bool coop = n_items <= coop_items(tree != nullptr);
+  // (the plan's two ranges, of up to two tokens and of more, share one launch)
+  const bool coop = four_waves_an_item(n_items, n_small, window, tree != nullptr);
   if (tree && coop)  // a tree is launched directly with exact counts (never from a graph)
     hipLaunchKernelGGL(attn_tree_coop_kernel, dim3(n_items), dim3(64 * kCoopWaves), 0, s, q, k_pool, v_pool, kv_base,
                        kv_cap, window, Hq, items, partials, groups, n_groups, sinks, out, tree);

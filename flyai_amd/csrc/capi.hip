@@ -411,7 +411,8 @@ static int record_step(flyai_stage* st, const StepPlan& sp, const int32_t* count
       RUN(launch_attn(B16(st->o_qrot), L.k_pool, L.v_pool, base_d, cap_d, L.sinks,
                       L.sliding ? c.window : 0, c.n_q_heads,
                       reinterpret_cast<const flyai_attn_item*>(blob + sp.off_items[p]), sp.grid_items[p],
-                      sp.n_small[p], reinterpret_cast<const flyai_attn_group*>(blob + sp.off_groups[p]),
+                      sp.lean[p] ? sp.grid_items[p] : sp.n_small[p],
+                      reinterpret_cast<const flyai_attn_group*>(blob + sp.off_groups[p]),
                       sp.grid_groups[p], counts ? counts + 2 * p : nullptr, F32(st->o_parts),
                       B16(st->o_attn), tree_d, sp.merge[p] != 0, s));
       RUN(launch_attn_prefill(B16(st->o_qrot), L.k_pool, L.v_pool, base_d, cap_d, L.sinks,

@@ -558,14 +558,9 @@ def test_attention_few_items_equal_many_items_bit_exact(window, split):
     assert torch.isfinite(many.float()).all()
 
 
-@pytest.mark.parametrize("window", [0, 128])
-@pytest.mark.parametrize("q_len", [1, 2, 4])
-def test_attention_item_count_rules_bit_exact(q_len, window):
-    """The launch's item count decides how many waves take an item and up to how many blocks one wave takes it
-    alone (one workgroup a CU, two a CU, more): the same sequences in launches on both sides of every line, with
-    key counts at both sides of every block line, give the same bits."""
+def _attention_item_count_rules(q_len, window, S, few_counts):
     from flyai_amd import ops
-    Hq, Hkv, D, cap, S = 64, 8, 64, 640, 72
+    Hq, Hkv, D, cap = 64, 8, 64, 640
     cus = torch.cuda.get_device_properties(0).multi_processor_count
     starts = [(64 * (1 + b % 9) + (b % 5) - 2) - q_len for b in range(S)]
     slab = Hkv * cap * D
@@ -588,11 +583,28 @@ def test_attention_item_count_rules_bit_exact(q_len, window):
         return out.view(torch.int16), len(items)
 
     many, n_many = run(S)
-    assert n_many > 2 * cus and torch.isfinite(many.view(torch.bfloat16).float()).all()
-    for n in (1, cus // 8, cus // 8 + 1, cus // 4, cus // 4 + 1):
+    assert n_many > 2 * cus and n_many == 8 * S and torch.isfinite(many.view(torch.bfloat16).float()).all()
+    for n in few_counts(cus):
         few, n_items = run(n)
         assert n_items == 8 * n
         assert torch.equal(few, many[:n * q_len]), n
+
+
+@pytest.mark.parametrize("window", [0, 128])
+@pytest.mark.parametrize("q_len", [1, 2, 4])
+def test_attention_item_count_rules_bit_exact(q_len, window):
+    """The launch's item count decides how many waves take an item and up to how many blocks one wave takes it
+    alone (one workgroup a CU, two a CU, more): the same sequences in launches on both sides of every line, with
+    key counts at both sides of every block line, give the same bits."""
+    _attention_item_count_rules(q_len, window, 72, lambda cus: (1, cus // 8, cus // 8 + 1, cus // 4, cus // 4 + 1))
+
+
+@pytest.mark.parametrize("q_len", [1, 2, 4])
+@pytest.mark.parametrize("window", [0, 128, 129])
+def test_attention_full_and_sliding_lines_bit_exact(window, q_len):
+    """The lines that depend on the layer: a full layer's items stay with four waves up to two and a half workgroups a
+    CU; a sliding layer's go to one wave where its window holds every item in the blocks one wave takes."""
+    _attention_item_count_rules(q_len, window, 100, lambda cus: (2, cus // 4, 5 * cus // 16, 5 * cus // 16 + 1))
 
 
 def test_attention_ignores_unwritten_nan_slots():
