@@ -1223,11 +1223,12 @@ inline bool use_dense(int rows_total, int E) { return (int64_t)rows_total >= (in
 // 128 experts, H = I = 2880, even routing, without / with it: 5 rows 293 / 306, 6 rows 318 / 302, 8 374 / 312, 12 386 / 330,
 // 18 382 / 357, 19 384 / 360, 20 389 / 414, 22 395 / 426: from 20 rows on a group or two pass 32 rows, and a second pass's units
 // start another round of workgroups.  With half of the rows on a tenth of the experts: 6 rows 424 / 365, 8 368 / 373,
-// 10.4 358 / 386, 12 362 / 390, 14 414 / 405, 18 469 / 423: from 8 to 13 rows it loses 1 to 8 % there (the other groups have
-// 4 to 8 rows, the row pass's best) and wins 17 to 21 % on even batches, and the host sees only the average.  Leaving
+// 10.4 358 / 386, 12 362 / 390, 14 414 / 405, 18 469 / 423; 64 experts 8 rows 188 / 197, 12 rows 189 / 207, 16 rows 222 /
+// 216; 32 and 256 experts win throughout.  From 8 to 13 rows it loses 1 to 10 % there (the other groups have 4 to 8 rows,
+// the row pass's best) and wins 15 to 23 % on even batches, and the host sees only the average.  Leaving
 // groups over 32 rows to the 96-row GEMM costs even batches 3 % and skewed ones of 32 experts 30 %.
 // Where the kernel's units of one block fill less than half of the CUs it starts at kMidFewFrom: 4 experts of 6 rows 28.6
-// without, 35.1 with it, 12 rows 43.8 / 35.2; 8 experts' down of 6 rows 13.7 / 17.7, of 8 32.6 / 17.7.
+// without, 35.1 with it, 8 rows 32.5 / 35.2, 12 rows 43.8 / 35.2; 8 experts' down of 6 rows 13.7 / 17.7, of 8 32.6 / 17.7.
 constexpr int kMidFrom = 6, kMidFewFrom = 8, kMidTo = 18;
 
 inline bool use_mid(int rows_total, int E, int N, int K) {
